@@ -74,6 +74,7 @@ EXPORTED_SYMBOLS = (
     "fuseml_gemm_epilogue",
     "fuseml_gemm_epilogue_supported",
     "fuseml_gemm_epilogue_config",
+    "fuseml_gemm_epilogue_ksplit",
     "fuseml_gemm_epilogue_force_variant",
     "fuseml_gemm_epilogue_chain",
     "fuseml_last_error",
@@ -194,6 +195,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.fuseml_gemm_epilogue_supported.restype = ctypes.c_int
     lib.fuseml_gemm_epilogue_config.argtypes = [desc_p, ctypes.POINTER(ctypes.c_int32)]
     lib.fuseml_gemm_epilogue_config.restype = ctypes.c_int
+    lib.fuseml_gemm_epilogue_ksplit.argtypes = [desc_p, ctypes.POINTER(ctypes.c_int32)]
+    lib.fuseml_gemm_epilogue_ksplit.restype = ctypes.c_int
     lib.fuseml_gemm_epilogue_force_variant.argtypes = [ctypes.c_char_p]
     lib.fuseml_gemm_epilogue_force_variant.restype = ctypes.c_int
     lib.fuseml_gemm_epilogue_chain.argtypes = [desc_p]

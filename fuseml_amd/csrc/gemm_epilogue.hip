@@ -109,7 +109,7 @@ int match_fixed_chain(const fuseml_gemm_desc& d);
 // 128x128 tiles (58.2; 64x128 63.8); 64x65536x4096 138.7 -> 125,
 // 16x65536x1024 36.0 -> 23.0, 128x65536x1024 38.7 -> 31.9 and 128x65536x4096
 // 151.9 -> 136.1 on lock-step tiles instead of 256x256 ones.
-TileConfig choose_partial_round(const fuseml_gemm_desc& d, int cus) {
+TileConfig choose_partial_round(const fuseml_gemm_desc& d, int cus, int64_t* least = nullptr) {
   struct Cand {
     const TileConfig* c;
     int w_one, w_two;  // weight with at most one / with two workgroups on a CU
@@ -128,8 +128,12 @@ TileConfig choose_partial_round(const fuseml_gemm_desc& d, int cus) {
       best_work = work;
     }
   }
+  if (least != nullptr) *least = best_work;
   return *best;
 }
+
+// Decode-sized M against a wide weight: a 128-column tile per CU or more.
+bool weight_streaming(const fuseml_gemm_desc& d, int cus) { return d.M <= 128 && cdiv(d.N, 128) >= cus; }
 
 // `cus`: the device's CU count (the 256-wide variants run one workgroup per CU).
 // `d` has its flags derived (derive_flags).
@@ -171,7 +175,7 @@ TileConfig choose_config(const fuseml_gemm_desc& d, int cus) {
   // 215.8 us and 128x32768x4096 59.6 -> 53.6 on the 128x128 tile at BK = 64
   // instead of 32 (eager 219.9 and 57.3); 64 and 16 rows: 113.0 and 41.8 on
   // 64x128 and 32x128 tiles (eager 134.2, 44.4).
-  if (d.M <= 128 && cdiv(d.N, 128) >= cus) return d.M <= 32 ? kNarrow32 : d.M <= 64 ? kNarrow64 : kSmall64;
+  if (weight_streaming(d, cus)) return d.M <= 32 ? kNarrow32 : d.M <= 64 ? kNarrow64 : kSmall64;
   const int64_t large_tiles = cdiv(d.M, 256) * cdiv(d.N, 256);
   if (2 * large_tiles <= cus || d.M <= 128) return choose_partial_round(d, cus);
   if (d.K % 64 == 0 && (d.K >= 8192 || (d.K >= 2048 && large_tiles >= cus))) return kDeep3;
@@ -180,6 +184,48 @@ TileConfig choose_config(const fuseml_gemm_desc& d, int cus) {
     if (ch != kChainGeneric && ch != kChainBiasGeluErf) return kDeep3;
   }
   return d.K >= 8192 ? kDeep : kLarge;
+}
+
+// The K-split tile (index into kKsplit) a launch of `d` runs on, or -1 for the
+// tiled family.  Both sides are priced in microseconds by what was measured on
+// 326 shapes of 1 to 2048 rows, 256 to 16384 columns and K = 256 to 16384 (bf16,
+// bias + residual), where the tiled family would run one of its tiles below a
+// round:
+//   K-split  3.5 + r (0.6 to 1.2 + 0.32 (mb + nb) K / 1024), r = tiles per CU, at
+//            least 1: launch, first loads, partials and epilogue, then operand
+//            bytes.  The 96 KB rings of the 32x64 and 64x32 tiles leave one
+//            workgroup per CU, so a further round overlaps nothing: 1 + r (5.1 + ..).
+//   tiled    -3 + work (5.05 + 3.6 K / 1024) / 160, work as choose_partial_round
+//            weighs it.
+// Each is within 8% of the measurement on average, 33% at worst, so the K-split
+// kernel runs where it is priced at 0.85 of the other or less: 227 of the 326
+// shapes, 2.0x faster there (geometric mean; 0.15-0.97 of the tiled time), e.g.
+// 8x4096x16384 107.7 -> 27.0, 64x4096x4096 31.4 -> 14.3, 128x256x1024 10.3 -> 5.1.
+// Not at 1024x1024x1024 (11.0 tiled, 13.0 here: operands shared by more waves
+// win) nor where the weight streams through a full row of tiles
+// (16x65536x1024 28.5 against 30.7).
+int choose_ksplit(const fuseml_gemm_desc& d, int cus) {
+  if (forced_variant() != 0 || d.K <= 0 || weight_streaming(d, cus)) return -1;
+  if (d.M > 128 && 2 * cdiv(d.M, 256) * cdiv(d.N, 256) > cus) return -1;
+  const double k = (double)d.K / 1024.0;
+  int best = -1;
+  double cost = 0.0;
+  for (int i = 0; i < kNumKsplit; ++i) {
+    const KsplitConfig& c = kKsplit[i];
+    const double tiles = (double)(cdiv(d.M, c.bm()) * cdiv(d.N, c.bn()));
+    const double r = tiles > cus ? tiles / cus : 1.0;
+    const bool alone = c.lds_bytes() > 80 * 1024;
+    const double fixed = alone ? 5.1 : c.mb * c.nb == 2 ? 0.6 : 1.2;
+    const double t = (alone ? 1.0 : 3.5) + r * (fixed + 0.32 * (c.mb + c.nb) * k);
+    if (best < 0 || t < cost) {
+      best = i;
+      cost = t;
+    }
+  }
+  int64_t work = 0;
+  choose_partial_round(d, cus, &work);
+  const double tiled = -3.0 + (double)work / (5.0 * 160.0) * (5.05 + 3.6 * k);
+  return cost < 0.85 * tiled ? best : -1;
 }
 
 bool check_output(const fuseml_output& o, const fuseml_gemm_desc& d, const char* what) {
@@ -528,6 +574,24 @@ int fuseml_gemm_epilogue_config(const fuseml_gemm_desc* desc, int32_t cfg[4]) {
   return FUSEML_OK;
 }
 
+int fuseml_gemm_epilogue_ksplit(const fuseml_gemm_desc* desc, int32_t cfg[4]) {
+  g_last_error[0] = '\0';
+  const int rc = validate(desc);
+  if (rc != FUSEML_OK) return rc;
+  int dev = 0, cus = 256;
+  if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices) {
+    const int known = g_device_cus[dev].load(std::memory_order_relaxed);
+    if (known > 0) cus = known;
+  }
+  const int i = choose_ksplit(*desc, cus);
+  if (i < 0) return 0;
+  cfg[0] = kKsplit[i].bm();
+  cfg[1] = kKsplit[i].bn();
+  cfg[2] = kKsplit[i].waves;
+  cfg[3] = kKsplit[i].lds_bytes();
+  return 1;
+}
+
 int fuseml_gemm_epilogue_chain(const fuseml_gemm_desc* desc) {
   g_last_error[0] = '\0';
   const int rc = validate(desc);
@@ -603,6 +667,15 @@ int fuseml_gemm_epilogue(const fuseml_gemm_desc* desc, void* stream_ptr) {
     }
   }
 
+  const int ks = choose_ksplit(d, cus);
+  if (ks >= 0) {
+    e = d.ab_dtype == FUSEML_BF16 ? launch_ksplit<__bf16>(d, ks, stream) : launch_ksplit<_Float16>(d, ks, stream);
+    if (e != hipSuccess) {
+      set_error("gemm_ksplit launch: %s", hipGetErrorString(e));
+      return FUSEML_EHIP;
+    }
+    return FUSEML_OK;
+  }
   const TileConfig c = choose_config(d, cus);
   const int ch = launch_chain(d, c);
   if (ch != kChainGeneric)

@@ -1,0 +1,4 @@
+// The K-split kernel's tiles for bf16 GEMM operands.
+#include "gemm_ksplit.h"
+
+template hipError_t fuseml_gemm::launch_ksplit<__bf16>(const fuseml_gemm_desc&, int, hipStream_t);

@@ -155,8 +155,16 @@ int fuseml_gemm_epilogue_supported(const fuseml_gemm_desc* desc);
 
 /* Tile configuration the library would launch for `desc`: writes BM, BN,
  * waves per workgroup and LDS bytes into cfg[0..3].  Replaces the launch
- * parameter selection of kernel_launcher.py:134-306 / sram_autotuner.py. */
+ * parameter selection of kernel_launcher.py:134-306 / sram_autotuner.py.  It
+ * speaks for the tiled family; a small output may run on the K-split kernel
+ * instead (fuseml_gemm_epilogue_ksplit). */
 int fuseml_gemm_epilogue_config(const fuseml_gemm_desc* desc, int32_t cfg[4]);
+
+/* Whether a launch of `desc` runs on the K-split kernel (few output tiles, the
+ * waves of a workgroup splitting K): 1 and its BM, BN, waves per workgroup and
+ * LDS bytes in cfg[0..3], 0 if it runs on the tiled family, a negative
+ * FUSEML_E* code for an invalid descriptor.  Never while a variant is pinned. */
+int fuseml_gemm_epilogue_ksplit(const fuseml_gemm_desc* desc, int32_t cfg[4]);
 
 /* The epilogue a launch of `desc` would compile in: 0 for the generic op loop
  * (the descriptor's ops interpreted at run time), else the id of the fixed
