@@ -74,6 +74,8 @@ EXPORTED_SYMBOLS = (
     "fuseml_gemm_epilogue",
     "fuseml_gemm_epilogue_supported",
     "fuseml_gemm_epilogue_config",
+    "fuseml_gemm_epilogue_f32",
+    "fuseml_gemm_epilogue_f32_supported",
     "fuseml_gemm_epilogue_ksplit",
     "fuseml_gemm_epilogue_force_variant",
     "fuseml_gemm_epilogue_chain",
@@ -195,6 +197,10 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.fuseml_gemm_epilogue_supported.restype = ctypes.c_int
     lib.fuseml_gemm_epilogue_config.argtypes = [desc_p, ctypes.POINTER(ctypes.c_int32)]
     lib.fuseml_gemm_epilogue_config.restype = ctypes.c_int
+    lib.fuseml_gemm_epilogue_f32.argtypes = [desc_p, ctypes.c_void_p]
+    lib.fuseml_gemm_epilogue_f32.restype = ctypes.c_int
+    lib.fuseml_gemm_epilogue_f32_supported.argtypes = [desc_p]
+    lib.fuseml_gemm_epilogue_f32_supported.restype = ctypes.c_int
     lib.fuseml_gemm_epilogue_ksplit.argtypes = [desc_p, ctypes.POINTER(ctypes.c_int32)]
     lib.fuseml_gemm_epilogue_ksplit.restype = ctypes.c_int
     lib.fuseml_gemm_epilogue_force_variant.argtypes = [ctypes.c_char_p]

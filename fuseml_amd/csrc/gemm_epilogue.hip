@@ -204,28 +204,52 @@ TileConfig choose_config(const fuseml_gemm_desc& d, int cus) {
 // Not at 1024x1024x1024 (11.0 tiled, 13.0 here: operands shared by more waves
 // win) nor where the weight streams through a full row of tiles
 // (16x65536x1024 28.5 against 30.7).
-int choose_ksplit(const fuseml_gemm_desc& d, int cus) {
-  if (forced_variant() != 0 || d.K <= 0 || weight_streaming(d, cus)) return -1;
-  if (d.M > 128 && 2 * cdiv(d.M, 256) * cdiv(d.N, 256) > cus) return -1;
-  const double k = (double)d.K / 1024.0;
+// The K-split tile (index into kKsplit) with the least priced time: `per_k` us
+// per block row or column and 1024 of K.
+int cheapest_ksplit(const fuseml_gemm_desc& d, int cus, double per_k, double* least) {
   int best = -1;
-  double cost = 0.0;
   for (int i = 0; i < kNumKsplit; ++i) {
     const KsplitConfig& c = kKsplit[i];
     const double tiles = (double)(cdiv(d.M, c.bm()) * cdiv(d.N, c.bn()));
     const double r = tiles > cus ? tiles / cus : 1.0;
     const bool alone = c.lds_bytes() > 80 * 1024;
     const double fixed = alone ? 5.1 : c.mb * c.nb == 2 ? 0.6 : 1.2;
-    const double t = (alone ? 1.0 : 3.5) + r * (fixed + 0.32 * (c.mb + c.nb) * k);
-    if (best < 0 || t < cost) {
+    const double t = (alone ? 1.0 : 3.5) + r * (fixed + per_k * (c.mb + c.nb) * (double)d.K / 1024.0);
+    if (best < 0 || t < *least) {
       best = i;
-      cost = t;
+      *least = t;
     }
   }
+  return best;
+}
+
+int choose_ksplit(const fuseml_gemm_desc& d, int cus) {
+  if (forced_variant() != 0 || d.K <= 0 || weight_streaming(d, cus)) return -1;
+  if (d.M > 128 && 2 * cdiv(d.M, 256) * cdiv(d.N, 256) > cus) return -1;
+  double cost = 0.0;
+  const int best = cheapest_ksplit(d, cus, 0.32, &cost);
   int64_t work = 0;
   choose_partial_round(d, cus, &work);
-  const double tiled = -3.0 + (double)work / (5.0 * 160.0) * (5.05 + 3.6 * k);
+  const double tiled = -3.0 + (double)work / (5.0 * 160.0) * (5.05 + 3.6 * (double)d.K / 1024.0);
   return cost < 0.85 * tiled ? best : -1;
+}
+
+// The K-split tile for fp32 GEMM operands, or -1 where splitting them into bf16
+// parts first (fuseml_split_bf16x3, three launches, 10 bytes of traffic per
+// element before the GEMM) is the faster way.  The K-split kernel reads 4 bytes
+// per element once and splits each fragment in registers, but every tile splits
+// its rows anew, at about 0.9 us per block and 1024 of K: it wins while the
+// output is small.  Measured (M x N x K, us, split passes and GEMM -> this):
+// 64x2048x512 15.9 -> 6.3, 1024x1024x1024 31 -> 22, 1024x1024x4096 80 -> 64,
+// 512x4096x256 23.8 -> 21.9, a tie at 2048x1024x1024 (38.0 and 39.0), and
+// 2048x2048x512 38.3 -> 52.7 the other way.
+int choose_ksplit_f32(const fuseml_gemm_desc& d, int cus) {
+  if (d.K <= 0) return -1;
+  double cost = 0.0;
+  const int best = cheapest_ksplit(d, cus, 0.9, &cost);
+  const KsplitConfig& c = kKsplit[best];
+  const int64_t padded = cdiv(d.M, c.bm()) * c.bm() * cdiv(d.N, c.bn()) * c.bn();
+  return d.M <= 32 || padded <= ((int64_t)1 << (d.K <= 512 ? 21 : 20)) ? best : -1;
 }
 
 bool check_output(const fuseml_output& o, const fuseml_gemm_desc& d, const char* what) {
@@ -241,7 +265,8 @@ bool check_output(const fuseml_output& o, const fuseml_gemm_desc& d, const char*
   return true;
 }
 
-int validate(const fuseml_gemm_desc* dp) {
+// `f32`: fp32 GEMM operands (fuseml_gemm_epilogue_f32) instead of 16-bit ones.
+int validate(const fuseml_gemm_desc* dp, bool f32 = false) {
   if (dp == nullptr) {
     set_error("null descriptor");
     return FUSEML_EINVAL;
@@ -256,7 +281,11 @@ int validate(const fuseml_gemm_desc* dp) {
     set_error("problem dimension exceeds 2^30");
     return FUSEML_EUNSUPPORTED;
   }
-  if (d.ab_dtype != FUSEML_BF16 && d.ab_dtype != FUSEML_F16) {
+  if (f32 && d.ab_dtype != FUSEML_F32) {
+    set_error("GEMM operand dtype %d: fp32 only", d.ab_dtype);
+    return FUSEML_EUNSUPPORTED;
+  }
+  if (!f32 && d.ab_dtype != FUSEML_BF16 && d.ab_dtype != FUSEML_F16) {
     set_error("GEMM operand dtype %d has no MFMA variant (bf16/f16 only)", d.ab_dtype);
     return FUSEML_EUNSUPPORTED;
   }
@@ -264,11 +293,12 @@ int validate(const fuseml_gemm_desc* dp) {
     set_error("null GEMM operand");
     return FUSEML_EINVAL;
   }
-  if (d.K > 0 && (d.K % 8 != 0 || d.lda % 8 != 0 || d.ldb % 8 != 0 || ((uintptr_t)d.a & 15) ||
+  const int eb = f32 ? 4 : 2, unit = 16 / eb;  // a 16-byte piece of a row
+  if (d.K > 0 && (d.K % unit != 0 || d.lda % unit != 0 || d.ldb % unit != 0 || ((uintptr_t)d.a & 15) ||
       ((uintptr_t)d.b & 15))) {
-    set_error("GEMM operands need K, lda, ldb multiples of 8 and 16-byte aligned bases "
+    set_error("GEMM operands need K, lda, ldb multiples of %d and 16-byte aligned bases "
               "(K=%lld lda=%lld ldb=%lld)",
-              (long long)d.K, (long long)d.lda, (long long)d.ldb);
+              unit, (long long)d.K, (long long)d.lda, (long long)d.ldb);
     return FUSEML_EUNSUPPORTED;
   }
   if (d.K > 0 && (d.lda < d.K || d.ldb < d.K)) {
@@ -278,7 +308,7 @@ int validate(const fuseml_gemm_desc* dp) {
   // Buffer resources are based at each tile's origin: the rows one tile reads
   // must span less than 2 GiB (the whole operand may be larger).
   const int64_t tm = d.M < kTileSpan ? d.M : kTileSpan, tn = d.N < kTileSpan ? d.N : kTileSpan;
-  if (d.K > 0 && (((tm - 1) * d.lda + d.K) * 2 >= kMaxBytes || ((tn - 1) * d.ldb + d.K) * 2 >= kMaxBytes)) {
+  if (d.K > 0 && (((tm - 1) * d.lda + d.K) * eb >= kMaxBytes || ((tn - 1) * d.ldb + d.K) * eb >= kMaxBytes)) {
     set_error("GEMM operand rows of one tile span 2 GiB or more (lda=%lld ldb=%lld)", (long long)d.lda,
               (long long)d.ldb);
     return FUSEML_EUNSUPPORTED;
@@ -592,6 +622,22 @@ int fuseml_gemm_epilogue_ksplit(const fuseml_gemm_desc* desc, int32_t cfg[4]) {
   return 1;
 }
 
+int fuseml_gemm_epilogue_f32_supported(const fuseml_gemm_desc* desc) {
+  g_last_error[0] = '\0';
+  const int rc = validate(desc, true);
+  if (rc != FUSEML_OK) return 0;
+  int dev = 0, cus = 256;
+  if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices) {
+    const int known = g_device_cus[dev].load(std::memory_order_relaxed);
+    if (known > 0) cus = known;
+  }
+  // Under a pinned variant, fp32 groups are to run on it: as split parts.  (A
+  // launch is not refused for that: its caller may have asked before the pin.)
+  if (forced_variant() == 0 && choose_ksplit_f32(*desc, cus) >= 0) return 1;
+  set_error("fp32 operands of this size run as bf16 parts (fuseml_split_bf16x3)");
+  return 0;
+}
+
 int fuseml_gemm_epilogue_chain(const fuseml_gemm_desc* desc) {
   g_last_error[0] = '\0';
   const int rc = validate(desc);
@@ -634,11 +680,13 @@ int fuseml_device_arch(int device, char* buf, int buflen) {
   return FUSEML_OK;
 }
 
-int fuseml_gemm_epilogue(const fuseml_gemm_desc* desc, void* stream_ptr) {
+// The start of a launch, common to both operand kinds: the validated descriptor
+// with its derived flags, the CU count, and the reduction buffers' fill on the
+// stream.  FUSEML_OK or an error code (the error is set).
+static int begin_launch(const fuseml_gemm_desc* desc, bool f32, hipStream_t stream, fuseml_gemm_desc& d, int& cus) {
   g_last_error[0] = '\0';
-  int rc = validate(desc);
+  const int rc = validate(desc, f32);
   if (rc != FUSEML_OK) return rc;
-  hipStream_t stream = reinterpret_cast<hipStream_t>(stream_ptr);
 
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
@@ -646,12 +694,16 @@ int fuseml_gemm_epilogue(const fuseml_gemm_desc* desc, void* stream_ptr) {
     set_error("hipGetDevice: %s", hipGetErrorString(e));
     return FUSEML_EHIP;
   }
-  const int cus = device_cus(dev);
+  cus = device_cus(dev);
   if (cus <= 0) return cus < 0 ? cus : FUSEML_EHIP;
 
-  fuseml_gemm_desc d = *desc;
+  d = *desc;
   fold_final_store(d);
   derive_flags(d);
+  if (f32 && choose_ksplit_f32(d, cus) < 0) {
+    set_error("fp32 operands of this size run as bf16 parts (fuseml_split_bf16x3)");
+    return FUSEML_EUNSUPPORTED;
+  }
 
   if (d.reduce_mask) {
     const int len = (int)(d.reduce_axis == 1 ? d.M : d.N);
@@ -666,6 +718,30 @@ int fuseml_gemm_epilogue(const fuseml_gemm_desc* desc, void* stream_ptr) {
       return FUSEML_EHIP;
     }
   }
+  return FUSEML_OK;
+}
+
+int fuseml_gemm_epilogue_f32(const fuseml_gemm_desc* desc, void* stream_ptr) {
+  hipStream_t stream = reinterpret_cast<hipStream_t>(stream_ptr);
+  fuseml_gemm_desc d;
+  int cus = 0;
+  const int rc = begin_launch(desc, true, stream, d, cus);
+  if (rc != FUSEML_OK) return rc;
+  const hipError_t e = launch_ksplit<float>(d, choose_ksplit_f32(d, cus), stream);
+  if (e != hipSuccess) {
+    set_error("gemm_ksplit launch: %s", hipGetErrorString(e));
+    return FUSEML_EHIP;
+  }
+  return FUSEML_OK;
+}
+
+int fuseml_gemm_epilogue(const fuseml_gemm_desc* desc, void* stream_ptr) {
+  hipStream_t stream = reinterpret_cast<hipStream_t>(stream_ptr);
+  fuseml_gemm_desc d;
+  int cus = 0;
+  const int rc = begin_launch(desc, false, stream, d, cus);
+  if (rc != FUSEML_OK) return rc;
+  hipError_t e = hipSuccess;
 
   const int ks = choose_ksplit(d, cus);
   if (ks >= 0) {

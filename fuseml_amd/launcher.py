@@ -111,6 +111,11 @@ class _Plan:
     and for each operand slot the input it comes from and whether it must be
     rebuilt per call (a dtype conversion or a broadcast that merging copies).
 
+    ``direct``: fp32 operands the library multiplies as they are
+    (``fuseml_gemm_epilogue_f32``: a small output, K-major rows); a call whose
+    bases are not 16-byte aligned takes ``split_plan``, the same signature's
+    plan on split operands.
+
     ``fast``: a call needs only the pointers (no negative strides, no operand
     rebuilt per call, no fp32 split, a non-empty output), written through
     ``words``, the descriptor as uint64 words; ``a_ok`` / ``b_ok``: the GEMM
@@ -118,7 +123,8 @@ class _Plan:
     alignment is still checked per call)."""
 
     __slots__ = ("desc", "M", "N", "K", "neg", "operands", "nbytes", "k_split", "fast", "words", "desc_ref",
-                 "a_ok", "b_ok", "lda", "ldb", "op_words", "red_words", "extra_words", "single_tile")
+                 "a_ok", "b_ok", "lda", "ldb", "op_words", "red_words", "extra_words", "single_tile", "direct",
+                 "split_plan")
 
     def __init__(self) -> None:
         self.desc = _abi.GemmDesc()
@@ -138,6 +144,8 @@ class _Plan:
         self.red_words: List[Tuple[int, str]] = []    # (descriptor word, reduction name)
         self.extra_words: List[int] = []
         self.single_tile = False
+        self.direct = False
+        self.split_plan: Optional["_Plan"] = None
 
 
 class HipKernelLauncher:
@@ -205,7 +213,7 @@ class HipKernelLauncher:
                 order.append(op.operand)
         return order
 
-    def _make_plan(self, inputs: Sequence[torch.Tensor]) -> _Plan:
+    def _make_plan(self, inputs: Sequence[torch.Tensor], allow_direct: bool = True) -> _Plan:
         spec = self.spec
         plan = _Plan()
         plan.neg = any(_has_negative_stride(inputs[i]) for i in self._used if isinstance(inputs[i], torch.Tensor))
@@ -271,9 +279,34 @@ class HipKernelLauncher:
         plan.red_words = [(_w_reduce(_abi.RED_SLOT[name]), name) for name in spec.reductions]
         plan.extra_words = [_w_extra(i) for i in range(len(spec.extra_dtypes))]
         plan.single_tile = spec.outputs == (("tile",),) and not spec.output_shapes and spec.store_tile
-        plan.fast = (not plan.neg and not plan.k_split and M > 0 and N > 0
-                     and not any(rebuild for _, rebuild in plan.operands))
+        ready = not plan.neg and M > 0 and N > 0 and not any(rebuild for _, rebuild in plan.operands)
+        if ready and plan.k_split and allow_direct and isinstance(self._lib, ctypes.CDLL):
+            self._try_direct(plan, inputs, a, b)
+        plan.fast = ready and not plan.k_split
         return plan
+
+    def _try_direct(self, plan: _Plan, inputs: Sequence[torch.Tensor], a: torch.Tensor, b: torch.Tensor) -> None:
+        """Turn an fp32 plan into a direct one if the library takes its
+        descriptor with the operands as they are."""
+        if a.stride(1) != 1 or b.stride(0) != 1:
+            return
+        probe = _abi.GemmDesc()
+        ctypes.memmove(ctypes.byref(probe), plan.desc_ref, ctypes.sizeof(probe))
+        probe.K, probe.ab_dtype, probe.lda, probe.ldb = plan.K, _abi.F32, a.stride(0), b.stride(1)
+        # any aligned addresses: the calls' own are checked per call
+        probe.a = probe.b = probe.out.ptr = 1 << 12
+        for i in range(probe.n_operands):
+            probe.operands[i].ptr = 1 << 12
+        for i in range(probe.n_extra):
+            probe.extra[i].ptr = 1 << 12
+        for slot in range(3):
+            probe.reduce_out[slot] = 1 << 12
+        if not self._lib.fuseml_gemm_epilogue_f32_supported(ctypes.byref(probe)):
+            return
+        plan.direct = plan.a_ok = plan.b_ok = True
+        plan.k_split = 0
+        plan.desc.K, plan.desc.ab_dtype = plan.K, _abi.F32
+        plan.lda, plan.ldb = a.stride(0), b.stride(1)
 
     def launch(self, *inputs: torch.Tensor) -> Any:
         """Allocate outputs, set the descriptor's pointers and call the C ABI."""
@@ -284,6 +317,10 @@ class HipKernelLauncher:
         if plan is None:
             plan = self._make_plan(inputs)
             self._plans[key] = plan
+        if plan.direct and (inputs[self.spec.left].data_ptr() | inputs[self.spec.right].data_ptr()) % 16:
+            if plan.split_plan is None:
+                plan.split_plan = self._make_plan(inputs, allow_direct=False)
+            plan = plan.split_plan
         # (tests may bind a recorder as the library: the general path, which
         # assumes no device, serves those)
         if plan.fast and self.timing_events is None and isinstance(self._lib, ctypes.CDLL):
@@ -339,7 +376,8 @@ class HipKernelLauncher:
                 t = torch.empty((red_len,), dtype=torch.float32, device=device)
                 w[wi] = t.data_ptr()
                 reds[name] = t
-        rc = self._lib.fuseml_gemm_epilogue(plan.desc_ref, torch._C._cuda_getCurrentRawStream(dev))
+        entry = self._lib.fuseml_gemm_epilogue_f32 if plan.direct else self._lib.fuseml_gemm_epilogue
+        rc = entry(plan.desc_ref, torch._C._cuda_getCurrentRawStream(dev))
         if rc != _abi.OK:
             raise _abi.FuseMLHipError(rc, _abi.last_error(self._lib))
         self.launch_count += 1
@@ -362,7 +400,7 @@ class HipKernelLauncher:
                 raise _abi.FuseMLHipError(
                     _abi.EINVAL, f"inputs on {sorted({str(inputs[i].device) for i in self._used})}: "
                     "every tensor must be on the launch's GPU")
-        if not plan.k_split:
+        if not plan.k_split and not plan.direct:
             a, b = _k_major_left(a), _k_major_right(b)
 
         tile = None
@@ -412,7 +450,8 @@ class HipKernelLauncher:
             else:
                 ev0, ev1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             ev0.record()
-        rc = self._lib.fuseml_gemm_epilogue(ctypes.byref(d), ctypes.c_void_p(stream))
+        entry = self._lib.fuseml_gemm_epilogue_f32 if plan.direct else self._lib.fuseml_gemm_epilogue
+        rc = entry(ctypes.byref(d), ctypes.c_void_p(stream))
         if rc != _abi.OK:
             raise _abi.FuseMLHipError(rc, _abi.last_error(self._lib))
         if timing is not None:

@@ -166,6 +166,18 @@ int fuseml_gemm_epilogue_config(const fuseml_gemm_desc* desc, int32_t cfg[4]);
  * FUSEML_E* code for an invalid descriptor.  Never while a variant is pinned. */
 int fuseml_gemm_epilogue_ksplit(const fuseml_gemm_desc* desc, int32_t cfg[4]);
 
+/* The same launch for fp32 GEMM operands (ab_dtype FUSEML_F32; K, lda, ldb
+ * multiples of 4, 16-byte aligned bases), as the three-term product of their
+ * bf16 parts (fuseml_split_bf16x3 below, whose parts it forms in registers).
+ * Built for outputs small enough that this beats splitting the operands first;
+ * FUSEML_EUNSUPPORTED for the others.  Replaces Triton's tf32 `tl.dot` on fp32
+ * inputs (fuseml/codegen/kernel_generator.py:1536). */
+int fuseml_gemm_epilogue_f32(const fuseml_gemm_desc* desc, void* stream);
+
+/* 1 if fuseml_gemm_epilogue_f32 accepts `desc`, 0 if not (reason in
+ * fuseml_last_error()).  Touches no device state. */
+int fuseml_gemm_epilogue_f32_supported(const fuseml_gemm_desc* desc);
+
 /* The epilogue a launch of `desc` would compile in: 0 for the generic op loop
  * (the descriptor's ops interpreted at run time), else the id of the fixed
  * chain kernel (1 none, 2 bias, 3 bias+GELU(erf), 4 bias+GELU(tanh),

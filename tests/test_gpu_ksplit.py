@@ -114,3 +114,53 @@ def test_ksplit_layouts_agree_with_the_tiled_kernels():
             finally:
                 _abi.force_variant(None)
             torch.testing.assert_close(got.float(), want.float(), rtol=2 ** -7, atol=2 ** -7)
+
+
+# fp32 operands multiplied as they are.
+F32_SHAPES = [(1, 8, 4), (64, 2048, 512), (17, 1030, 1004), (33, 257, 36), (31, 4099, 260), (500, 1023, 132),
+              (1000, 520, 516)]
+
+
+@pytest.mark.parametrize("chain", ["bias_gelu_tanh", "act_heavy", "scalars"])
+@pytest.mark.parametrize("shape", F32_SHAPES, ids=_ID)
+def test_fp32_direct_parity(shape, chain):
+    """Against the float64 oracle (1e-4, as every fp32 group), and no further
+    from it than the split passes' result of the same inputs: the same bf16
+    products, summed in fp32 in another order (1.5x, or 1e-6 of the result)."""
+    M, N, K = shape
+    a, w = _gemm_inputs(M, N, K, torch.float32, seed=51)
+    ops = _operands(M, N, torch.float32, seed=52)
+    inputs = ops + [a, w.t()]
+    left, right = len(ops), len(ops) + 1
+    print(f"case fp32 direct {shape} {chain}", flush=True)
+    L = _launcher(_spec(left=left, right=right, ops=CHAINS[chain], out_dtype=torch.float32), len(inputs))
+    dev = [t.cuda() for t in inputs]
+    got = _np(L(*dev))
+    (plan,) = L._plans.values()
+    assert plan.direct
+    # a base that is not 16-byte aligned takes the split passes
+    odd = torch.empty(M * K + 1, device="cuda")[1:].view(M, K).copy_(dev[left])
+    split = _np(L(*dev[:left], odd, dev[right]))
+    assert plan.split_plan is not None and not plan.split_plan.direct
+    ref = ora.gemm_epilogue([_np(t) for t in inputs], left, right, CHAINS[chain])["tile"]
+    assert np.isclose(got, ref, rtol=1e-4, atol=1e-4).all(), np.abs(got - ref).max()
+    norm = np.linalg.norm(ref)
+    assert np.linalg.norm(got - ref) <= 1.5 * np.linalg.norm(split - ref) + 1e-6 * norm
+
+
+def test_fp32_direct_non_finite_matches_the_split_passes():
+    """inf, NaN and values above the largest bf16 in both operands: NaN and inf
+    come out where the split passes put them, all else agrees to 1e-4."""
+    M, N, K = 40, 72, 100
+    a, w = _gemm_inputs(M, N, K, torch.float32, seed=53)
+    a[:, ::2] = torch.round(a[:, ::2] * 4) / 4 + 0.25
+    a[0, 1], a[3, K - 1], a[5, 50], a[7, 2] = float("inf"), -float("inf"), float("nan"), 3.4e38
+    w[2, 3], w[9, 1], w[11, 99] = float("inf"), float("nan"), -3.39e38
+    dev, wt = a.cuda(), w.cuda().t()
+    L = _launcher(_spec(left=0, right=1, ops=[("scale", -1, 0.5)], out_dtype=torch.float32), 2)
+    got = L(dev, wt)
+    (plan,) = L._plans.values()
+    assert plan.direct
+    want = L(torch.empty(M * K + 1, device="cuda")[1:].view(M, K).copy_(dev), wt)
+    torch.testing.assert_close(got, want, rtol=1e-4, atol=1e-4, equal_nan=True)
+    assert torch.isnan(got).any() and torch.isinf(got).any()

@@ -348,3 +348,25 @@ def test_host_tensors_are_refused_before_any_device_call():
     guarded = HipKernelLauncher(spec, 3, eager_fn=lambda bb, xx, ww: torch.relu(torch.addmm(bb, xx, ww)))
     out = guarded(b, x, w.t())
     assert guarded.fallback_count == 1 and torch.equal(out, torch.relu(torch.addmm(b, x, w.t())))
+
+
+@pytest.mark.parametrize("make_x,make_wt,direct", [
+    (lambda m, k: torch.randn(m, k), lambda n, k: torch.randn(n, k).t(), True),
+    (lambda m, k: torch.randn(m, k + 8)[:, :k], lambda n, k: torch.randn(n, k + 4)[:, :k].t(), True),
+    (lambda m, k: torch.randn(m, k + 1)[:, :k], lambda n, k: torch.randn(n, k).t(), False),   # rows not 16-byte aligned
+    (lambda m, k: torch.randn(k, m).t(), lambda n, k: torch.randn(n, k).t(), False),          # x not K-major
+    (lambda m, k: torch.randn(m, k), lambda n, k: torch.randn(k, n), False),                  # W not K-major
+    (lambda m, k: torch.randn(m, 2 * k)[:, ::2], lambda n, k: torch.randn(n, k).t(), False),  # strided K
+    (lambda m, k: torch.randn(1, k).expand(m, k), lambda n, k: torch.randn(n, k).t(), False),  # rows on top of each other
+    (lambda m, k: torch.randn(m, k - 1), lambda n, k: torch.randn(n, k - 1).t(), False),      # K % 4 != 0
+])
+def test_fp32_plan_is_direct_only_for_k_major_aligned_operands(make_x, make_wt, direct):
+    """The real library (host checks only): which fp32 layouts the K-split kernel
+    reads as they are; every other keeps the split passes' plan."""
+    M, N, K = 8, 24, 64
+    launcher = HipKernelLauncher(EpilogueSpec(0, 1, (EpiOp("relu"),), torch.float32), 2)
+    plan = launcher._make_plan((make_x(M, K), make_wt(N, K)))
+    assert (plan.direct, plan.k_split == 0, plan.fast) == (direct, direct, direct)
+    assert plan.desc.ab_dtype == (_abi.F32 if direct else _abi.BF16)
+    big = launcher._make_plan((torch.randn(4096, K), torch.randn(2048, K).t()))  # a large output: split passes
+    assert not big.direct and big.k_split == K
