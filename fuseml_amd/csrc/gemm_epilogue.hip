@@ -156,14 +156,16 @@ TileConfig choose_config(const fuseml_gemm_desc& d, int cus) {
   // to stay busy; below one full wave of 256-tile work the 128x128 variant
   // fills more CUs.  Of the 256x256 schedules, the one-wave-per-SIMD ones have
   // the faster K loop but the slower epilogue (no second wave on a SIMD to
-  // overlap its latencies).  The whole-stage one wins from K = 2048 with at
-  // least one full round of tiles (C4 2%, C5 4-10%, C2's second GEMM at K =
-  // 4096 and 256 tiles 3%) or from K = 8192.  At K = 1024 its generic op loop
-  // loses 12-16% on bias+GELU and C3's chain, but with a fixed-chain epilogue
-  // it wins on every fixed chain (3-7% on 256 to 1024 tiles; none, bias, ReLU,
-  // bias+ReLU, GELU(tanh), bias+residual, the act-heavy chain) except
-  // bias+GELU(erf), which ties or loses up to 1.5%.  With K % 64 != 0 the
-  // two-stage one takes over from K = 8192.
+  // overlap its latencies).  The whole-stage one's fixed-chain kernels win from
+  // K = 1024, on full rounds and on a partial one (136 to 224 tiles) alike: bf16
+  // ReLU, residual and act-heavy chains 0.94-1.01 of the ping-pong kernel's time
+  // at K = 1024 and 0.91-0.96 at K = 4096, fp16 ones 0.92-1.00 and 0.89-0.95
+  // (8192x4096x4096 bias+residual, fp16, 260 -> 231 us).  bias+GELU(erf), the
+  // chain with the most VALU work, only from K = 2048 (0.94-1.02 there, 0.92-0.97
+  // at K = 4096; 1.00-1.05 at K = 1024).  Its generic op loop loses 3-17% below
+  // K = 2048 and on partial rounds, and wins from K = 2048 with at least one
+  // full round of tiles or from K = 8192.  With K % 64 != 0 the two-stage one
+  // takes over from K = 8192.
   // Below one round of 256x256 tiles (2 x large_tiles <= cus) the smaller
   // tiles (choose_partial_round): at 128 large tiles on 256 CUs the 128x128
   // one was 7-17% faster than 256x256 (bias+GELU at K = 512-1024), from 144
@@ -179,9 +181,9 @@ TileConfig choose_config(const fuseml_gemm_desc& d, int cus) {
   const int64_t large_tiles = cdiv(d.M, 256) * cdiv(d.N, 256);
   if (2 * large_tiles <= cus || d.M <= 128) return choose_partial_round(d, cus);
   if (d.K % 64 == 0 && (d.K >= 8192 || (d.K >= 2048 && large_tiles >= cus))) return kDeep3;
-  if (d.K % 64 == 0 && d.K >= 1024 && large_tiles >= cus) {
+  if (d.K % 64 == 0 && d.K >= 1024) {
     const int ch = match_fixed_chain(d);
-    if (ch != kChainGeneric && ch != kChainBiasGeluErf) return kDeep3;
+    if (ch != kChainGeneric && (ch != kChainBiasGeluErf || d.K >= 2048)) return kDeep3;
   }
   return d.K >= 8192 ? kDeep : kLarge;
 }
@@ -427,12 +429,13 @@ void derive_flags(fuseml_gemm_desc& d) {
 
 // The fixed chain (FixedChain) that expresses the descriptor's epilogue, or
 // kChainGeneric.  Called after derive_flags: a "row" operand is a [N] vector
-// holding an LDS slot, a "tile" operand the LDS-staged bf16 2-D operand.
-// Fixed chains are built for bf16 GEMM operands, no escape stores, and no
-// reductions except after a lone relu (the ReLU + row/column reductions
-// group).
+// holding an LDS slot, a "tile" operand the LDS-staged 2-D operand of the GEMM
+// operands' type.  Fixed chains are built for bf16 GEMM operands and for fp16
+// ones with an fp16 output, no escape stores, and no reductions except after a
+// lone relu (the ReLU + row/column reductions group).
 int match_fixed_chain(const fuseml_gemm_desc& d) {
-  if (d.ab_dtype != FUSEML_BF16 || d.n_extra != 0) return kChainGeneric;
+  if (d.n_extra != 0 || (d.ab_dtype == FUSEML_F16 && d.out.ptr != nullptr && d.out.dtype != FUSEML_F16))
+    return kChainGeneric;
   auto is = [&](int o, int kind) { return o < d.n_ops && d.ops[o].kind == kind; };
   auto row = [&](int o) {
     if (!is(o, FUSEML_OP_ADD)) return false;
@@ -442,7 +445,7 @@ int match_fixed_chain(const fuseml_gemm_desc& d) {
   auto tile = [&](int o, int kind) {
     if (!is(o, kind)) return false;
     const fuseml_operand& op = d.operands[d.ops[o].operand];
-    return (op.reserved & kFlagStage) != 0 && op.dtype == FUSEML_BF16;
+    return (op.reserved & kFlagStage) != 0 && op.dtype == d.ab_dtype;
   };
   int ch = kChainGeneric;
   switch (d.n_ops) {
@@ -491,35 +494,35 @@ hipError_t launch_variant(const fuseml_gemm_desc& d, hipStream_t stream, int max
   return hipGetLastError();
 }
 
-// A fixed-chain kernel of variant C (bf16 operands; reductions only with
-// kChainRelu, as match_fixed_chain guarantees).
-template <const TileConfig& C, int CH>
+// A fixed-chain kernel of variant C (reductions only with kChainRelu, as
+// match_fixed_chain guarantees).
+template <const TileConfig& C, typename T, int CH>
 void launch_fixed_one(const fuseml_gemm_desc& d, hipStream_t stream, dim3 grid, dim3 block) {
   if constexpr (CH == kChainRelu) {
     if (d.reduce_mask != 0) {
-      hipLaunchKernelGGL((gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, C.sched, __bf16, true, CH>),
-                         grid, block, 0, stream, d);
+      hipLaunchKernelGGL((gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, C.sched, T, true, CH>), grid,
+                         block, 0, stream, d);
       return;
     }
   }
-  hipLaunchKernelGGL((gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, C.sched, __bf16, false, CH>),
-                     grid, block, 0, stream, d);
+  hipLaunchKernelGGL((gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, C.sched, T, false, CH>), grid,
+                     block, 0, stream, d);
 }
 
-template <const TileConfig& C>
+template <const TileConfig& C, typename T>
 hipError_t launch_fixed(const fuseml_gemm_desc& d, int ch, hipStream_t stream, int max_wg) {
   int64_t tiles = cdiv(d.M, C.bm) * cdiv(d.N, C.bn);
   if (max_wg > 0 && tiles > max_wg) tiles = max_wg;
   const dim3 grid((unsigned)tiles), block(C.wm * C.wn * 64);
   switch (ch) {
-    case kChainNone: launch_fixed_one<C, kChainNone>(d, stream, grid, block); break;
-    case kChainBias: launch_fixed_one<C, kChainBias>(d, stream, grid, block); break;
-    case kChainBiasGeluErf: launch_fixed_one<C, kChainBiasGeluErf>(d, stream, grid, block); break;
-    case kChainBiasGeluTanh: launch_fixed_one<C, kChainBiasGeluTanh>(d, stream, grid, block); break;
-    case kChainBiasRelu: launch_fixed_one<C, kChainBiasRelu>(d, stream, grid, block); break;
-    case kChainBiasTile: launch_fixed_one<C, kChainBiasTile>(d, stream, grid, block); break;
-    case kChainActHeavy: launch_fixed_one<C, kChainActHeavy>(d, stream, grid, block); break;
-    case kChainRelu: launch_fixed_one<C, kChainRelu>(d, stream, grid, block); break;
+    case kChainNone: launch_fixed_one<C, T, kChainNone>(d, stream, grid, block); break;
+    case kChainBias: launch_fixed_one<C, T, kChainBias>(d, stream, grid, block); break;
+    case kChainBiasGeluErf: launch_fixed_one<C, T, kChainBiasGeluErf>(d, stream, grid, block); break;
+    case kChainBiasGeluTanh: launch_fixed_one<C, T, kChainBiasGeluTanh>(d, stream, grid, block); break;
+    case kChainBiasRelu: launch_fixed_one<C, T, kChainBiasRelu>(d, stream, grid, block); break;
+    case kChainBiasTile: launch_fixed_one<C, T, kChainBiasTile>(d, stream, grid, block); break;
+    case kChainActHeavy: launch_fixed_one<C, T, kChainActHeavy>(d, stream, grid, block); break;
+    case kChainRelu: launch_fixed_one<C, T, kChainRelu>(d, stream, grid, block); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -755,7 +758,8 @@ int fuseml_gemm_epilogue(const fuseml_gemm_desc* desc, void* stream_ptr) {
   const TileConfig c = choose_config(d, cus);
   const int ch = launch_chain(d, c);
   if (ch != kChainGeneric)
-    e = launch_fixed<kDeep3>(d, ch, stream, cus);
+    e = d.ab_dtype == FUSEML_BF16 ? launch_fixed<kDeep3, __bf16>(d, ch, stream, cus)
+                                  : launch_fixed<kDeep3, _Float16>(d, ch, stream, cus);
   else if (c.sched == kDeep.sched)
     e = launch_variant<kDeep>(d, stream, cus);
   else if (c.sched == kLarge.sched && c.bn == kLarge128.bn)

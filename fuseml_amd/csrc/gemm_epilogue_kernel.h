@@ -1228,7 +1228,7 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
           static_for<0, 16>([&](auto r) { A[j][(int)r] = fmaf(a, x[r], A[j][(int)r]); });
         });
       };
-      // The staged bf16 tile's values of this block, all row blocks' 8-byte
+      // The staged tile's values of this block (of the GEMM operands' type), all row blocks' 8-byte
       // units read before any is used (32 registers).
       auto read_tile = [&](uint2(&wb)[NJ][4]) {
         const int u0 = (wn * TN + 32 * i) / 4 + khalf;
@@ -1241,7 +1241,10 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
       };
       auto tile_value = [&](const uint2(&wb)[NJ][4], auto j, auto r) {
         const uint32_t w = (r & 2) ? wb[j][r / 4].y : wb[j][r / 4].x;
-        return (r & 1) ? __uint_as_float(w & 0xffff0000u) : __uint_as_float(w << 16);
+        if constexpr (std::is_same<T, _Float16>::value)
+          return f16_bits_to_f32((r & 1) ? w >> 16 : w & 0xffffu);
+        else
+          return (r & 1) ? __uint_as_float(w & 0xffff0000u) : __uint_as_float(w << 16);
       };
       auto relu_all = [&]() {
         static_for<0, NJ>([&](auto j) {

@@ -62,7 +62,7 @@ hipError_t launch_ksplit(const fuseml_gemm_desc& d, int index, hipStream_t strea
 // runtime op loop; every other value is one fixed op sequence, matched on the
 // host (operand kinds included) and compiled as straight-line code with no
 // per-op dispatch.  "row" is a [N] vector operand in an LDS slot, "tile" the
-// LDS-staged bf16 2-D operand; ADD keeps its alpha from the descriptor.
+// LDS-staged 2-D operand of the GEMM operands' type; ADD keeps its alpha from the descriptor.
 enum FixedChain : int {
   kChainGeneric = 0,
   kChainNone = 1,          // (no ops)
