@@ -399,12 +399,9 @@ void derive_flags(fuseml_gemm_desc& d) {
     const int eb = op.dtype == FUSEML_F32 ? 4 : 2;
     const bool vec = op.stride_n == 1 && (op.stride_m % 4 == 0) && (d.N % 4 == 0) &&
                      ((uintptr_t)op.ptr % (4 * eb) == 0);
-    // Column reductions write their partials over the staging tile while other
-    // waves are still in the op chain, so they rule out a staged operand.
-    const bool stage = eb == 2 && op.stride_n == 1 && op.stride_m != 0 && (op.stride_m % 8 == 0) &&
-                       (d.N % 8 == 0) && ((uintptr_t)op.ptr % 16 == 0) &&
-                       !(d.reduce_mask != 0 && d.reduce_axis == 0);
-    op.reserved = (vec ? kFlagVec4 : 0) | (stage ? kFlagStage : 0);
+    const bool stage = eb == 2 && op.stride_n == 1 && op.stride_m != 0 && d.N >= 8;
+    const bool aligned = op.stride_m % 8 == 0 && d.N % 8 == 0 && (uintptr_t)op.ptr % 16 == 0;
+    op.reserved = (vec ? kFlagVec4 : 0) | (stage ? kFlagStage : 0) | (aligned ? kFlagAligned : 0);
   }
   // Vector operands of ADD/MUL ops get LDS slots, in first-use order.
   int slots = 0;
@@ -419,9 +416,9 @@ void derive_flags(fuseml_gemm_desc& d) {
   auto out_flags = [&](fuseml_output& o) {
     const int eb = o.dtype == FUSEML_F32 ? 4 : 2;
     const bool vec = o.ptr != nullptr && o.ld % 4 == 0 && d.N % 4 == 0 && (uintptr_t)o.ptr % (4 * eb) == 0;
-    const bool stage = o.ptr != nullptr && eb == 2 && o.ld % 8 == 0 && d.N % 8 == 0 &&
-                       (uintptr_t)o.ptr % 16 == 0;
-    o.reserved = (vec ? kFlagVec4 : 0) | (stage ? kFlagStage : 0);
+    const bool stage = o.ptr != nullptr && eb == 2 && d.N >= 8;
+    const bool aligned = o.ld % 8 == 0 && d.N % 8 == 0 && (uintptr_t)o.ptr % 16 == 0;
+    o.reserved = (vec ? kFlagVec4 : 0) | (stage ? kFlagStage : 0) | (aligned ? kFlagAligned : 0);
   };
   out_flags(d.out);
   for (int i = 0; i < d.n_extra; ++i) out_flags(d.extra[i]);
@@ -445,7 +442,7 @@ int match_fixed_chain(const fuseml_gemm_desc& d) {
   auto tile = [&](int o, int kind) {
     if (!is(o, kind)) return false;
     const fuseml_operand& op = d.operands[d.ops[o].operand];
-    return (op.reserved & kFlagStage) != 0 && op.dtype == d.ab_dtype;
+    return (op.reserved & kFlagStage) != 0 && (op.reserved & kFlagAligned) != 0 && op.dtype == d.ab_dtype;
   };
   int ch = kChainGeneric;
   switch (d.n_ops) {

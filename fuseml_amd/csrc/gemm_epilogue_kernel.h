@@ -234,6 +234,96 @@ __device__ __forceinline__ void store_out4(const Out& o, int m, int n, int M, in
   }
 }
 
+// The same for a lane's 16 values of a 32 x 32 block: four runs of 4 columns, 8
+// apart, from column nb of row m.  One uniform choice of the access kind per
+// block instead of per run: a quarter of the branches and code.
+template <typename Op>
+__device__ __forceinline__ void load_operand16(const Op& op, int m0, int n0, int m, int nb, int M, int N, float v[16]) {
+  const int dt = op.dtype;
+  const int eb = dtype_bytes(dt);
+  const __amdgpu_buffer_rsrc_t r =
+      make_rsrc_at(op.ptr, ((int64_t)m0 * op.stride_m + (int64_t)n0 * op.stride_n) * eb, op.extent * eb);
+  const int64_t row = (int64_t)(m - m0) * op.stride_m;
+  auto offset = [&](int n, int e) {
+    return m < M && n < N ? (uint32_t)((row + (int64_t)(n + e - n0) * op.stride_n) * eb) : kOOB;
+  };
+  if ((op.reserved & kFlagVec4) && dt == FUSEML_F32) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const i32x4_t x = __builtin_amdgcn_raw_buffer_load_b128(r, offset(nb + 8 * g, 0), 0, 0);
+      v[4 * g] = __int_as_float(x.x); v[4 * g + 1] = __int_as_float(x.y);
+      v[4 * g + 2] = __int_as_float(x.z); v[4 * g + 3] = __int_as_float(x.w);
+    }
+    return;
+  }
+  uint32_t bits[16];
+  if (op.reserved & kFlagVec4) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const i32x2_t x = __builtin_amdgcn_raw_buffer_load_b64(r, offset(nb + 8 * g, 0), 0, 0);
+      bits[4 * g] = (uint32_t)x.x & 0xffffu; bits[4 * g + 1] = (uint32_t)x.x >> 16;
+      bits[4 * g + 2] = (uint32_t)x.y & 0xffffu; bits[4 * g + 3] = (uint32_t)x.y >> 16;
+    }
+  } else if (eb == 4) {
+#pragma unroll
+    for (int q = 0; q < 16; ++q)
+      bits[q] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, offset(nb + 8 * (q >> 2), q & 3), 0, 0);
+  } else {
+#pragma unroll
+    for (int q = 0; q < 16; ++q)
+      bits[q] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(r, offset(nb + 8 * (q >> 2), q & 3), 0, 0) & 0xffffu;
+  }
+  if (dt == FUSEML_F32) {
+#pragma unroll
+    for (int q = 0; q < 16; ++q) v[q] = __uint_as_float(bits[q]);
+  } else if (dt == FUSEML_BF16) {
+#pragma unroll
+    for (int q = 0; q < 16; ++q) v[q] = bf16_bits_to_f32(bits[q]);
+  } else {
+#pragma unroll
+    for (int q = 0; q < 16; ++q) v[q] = f16_bits_to_f32(bits[q]);
+  }
+}
+
+template <typename Out, typename Acc>
+__device__ __forceinline__ void store_out16(const Out& o, int m, int nb, int M, int N, const Acc& v) {
+  if (m >= M) return;
+  const int64_t base = (int64_t)m * o.ld + nb;
+  if (o.dtype == FUSEML_F32) {
+    float* p = reinterpret_cast<float*>(o.ptr) + base;
+    if (o.reserved & kFlagVec4) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        if (nb + 8 * g < N)
+          *reinterpret_cast<float4*>(p + 8 * g) = make_float4(v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 16; ++q)
+        if (nb + 8 * (q >> 2) + (q & 3) < N) p[8 * (q >> 2) + (q & 3)] = v[q];
+    }
+    return;
+  }
+  uint32_t w[8];
+  if (o.dtype == FUSEML_BF16) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) w[q] = pack_bf16x2(v[2 * q], v[2 * q + 1]);
+  } else {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) w[q] = pack_f16x2(v[2 * q], v[2 * q + 1]);
+  }
+  uint16_t* p = reinterpret_cast<uint16_t*>(o.ptr) + base;
+  if (o.reserved & kFlagVec4) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      if (nb + 8 * g < N) *reinterpret_cast<uint2*>(p + 8 * g) = make_uint2(w[2 * g], w[2 * g + 1]);
+  } else {
+#pragma unroll
+    for (int q = 0; q < 16; ++q)
+      if (nb + 8 * (q >> 2) + (q & 3) < N)
+        p[8 * (q >> 2) + (q & 3)] = (uint16_t)(w[q >> 1] >> (16 * (q & 1)));
+  }
+}
+
 // Float atomic max through integer atomics, dispatched on the sign bit
 // (amax_order.h: -0.0 takes the unsigned-min path like every other value with
 // the sign bit set; NaN is written as 0x7fc00000 and then always kept).
@@ -290,6 +380,12 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
+}
+
+// The value of the lane whose index differs in bit DIST (within 32 lanes).
+template <int DIST>
+__device__ __forceinline__ float lane_xor(float x) {
+  return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(x), (DIST << 10) | 0x1f));
 }
 
 // Compile-time loop: f(std::integral_constant<int, I>) for I in [B, E).  Used
@@ -405,6 +501,29 @@ __device__ __forceinline__ int stage_chunk(int r, int c) {
 template <int BN>
 __device__ __forceinline__ bool stage_swapped(int r) {
   return !kChunkSwizzle<BN> && (r & 1);
+}
+
+// A 16-byte chunk at an address that is a multiple of 2 only: one global access
+// (memory instructions take any alignment here).  Rows of odd length or pitch go
+// through the staging tile with it like the others, where 2- and 8-byte accesses
+// from the accumulator layout (32 rows per instruction) doubled a kernel's time:
+// 4096x4095x1024 bias+GELU 82.2 -> 40.7 us, bias+residual 104.2 -> 49.9 (4096
+// columns: 42.9 and 40.3; the residual's rows are fetched after the K loop, not by
+// the DMA during it, which takes aligned chunks only).
+typedef int i32x4_any_t __attribute__((ext_vector_type(4), aligned(2)));
+
+// Elements [n, N) of a row (8 or more long) as a chunk whose first N - n < 8
+// elements are valid: the row's last 8 elements, moved down, so that nothing past
+// the row is read.
+__device__ __forceinline__ i32x4_t load_row_end(const uint16_t* row, int n, int N) {
+  const i32x4_t x = *reinterpret_cast<const i32x4_any_t*>(row + N - 8);
+  const int drop = n - (N - 8);  // 1 .. 7 elements
+  const uint64_t lo = (uint64_t)(uint32_t)x.x | ((uint64_t)(uint32_t)x.y << 32);
+  const uint64_t hi = (uint64_t)(uint32_t)x.z | ((uint64_t)(uint32_t)x.w << 32);
+  const int b = 16 * (drop & 3);
+  const uint64_t l = drop & 4 ? hi : lo, h = drop & 4 ? 0 : hi;
+  const uint64_t r0 = b ? (l >> b) | (h << (64 - b)) : l, r1 = h >> b;
+  return i32x4_t{(int)(uint32_t)r0, (int)(uint32_t)(r0 >> 32), (int)(uint32_t)r1, (int)(uint32_t)(r1 >> 32)};
 }
 
 __device__ __forceinline__ i32x4_t swap_halves(i32x4_t x) { return i32x4_t{x.z, x.w, x.x, x.y}; }
@@ -579,7 +698,7 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
     constexpr int RPS = STAGE / SP;   // staging rows per pipeline slot
     static_assert(!kOpDma || (STAGE % SP == 0 && RPS % 32 == 0 && RPS == RPD * NW * LPS),
                   "operand DMAs line up with the stage DMAs");
-    const bool op_dma = kOpDma && staged >= 0;
+    const bool op_dma = kOpDma && staged >= 0 && (d.operands[staged].reserved & kFlagAligned) != 0;
     const void* op_ptr = d.a;
     int64_t op_bytes = 0;  // bytes of the operand from its row m0 on
     uint32_t op_o[kOpDma ? LPS : 1];  // chunk c's byte offset in its slot (kOOB: column past N)
@@ -1154,19 +1273,50 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
       constexpr int NP = BM / RPP;
       constexpr int PB = NP < 8 ? NP : 8;
       static_assert(NP % PB == 0, "pass batches");
-      static_for<0, NP / PB>([&](auto b) {
-        i32x4_t x[PB];
-        static_for<0, PB>([&](auto q) {
-          const int rl = (b * PB + q) * RPP + crow;
-          const int m = m0 + rl, n = n0 + 8 * cchk;
-          const uint32_t o32 = ((uint32_t)rl * (uint32_t)osm + (uint32_t)n) * 2u;
-          x[q] = __builtin_amdgcn_raw_buffer_load_b128(r, (m < M && n < N) ? o32 : kOOB, 0, 0);
+      if (d.operands[staged].reserved & kFlagAligned) {
+        static_for<0, NP / PB>([&](auto b) {
+          i32x4_t x[PB];
+          static_for<0, PB>([&](auto q) {
+            const int rl = (b * PB + q) * RPP + crow;
+            const int m = m0 + rl, n = n0 + 8 * cchk;
+            const uint32_t o32 = ((uint32_t)rl * (uint32_t)osm + (uint32_t)n) * 2u;
+            x[q] = __builtin_amdgcn_raw_buffer_load_b128(r, (m < M && n < N) ? o32 : kOOB, 0, 0);
+          });
+          static_for<0, PB>([&](auto q) {
+            const int rl = (b * PB + q) * RPP + crow;
+            *reinterpret_cast<i32x4_t*>(stg + stage_chunk<BN>(rl, cchk)) =
+                stage_swapped<BN>(rl) ? swap_halves(x[q]) : x[q];
+          });
         });
-        static_for<0, PB>([&](auto q) {
-          const int rl = (b * PB + q) * RPP + crow;
-          *reinterpret_cast<i32x4_t*>(stg + stage_chunk<BN>(rl, cchk)) = stage_swapped<BN>(rl) ? swap_halves(x[q]) : x[q];
-        });
-      });
+      } else {
+        // Rows that are not whole 16-byte chunks at 16-byte addresses: each chunk
+        // by one access of any alignment, the row's last one from its end.  A
+        // runtime loop over batches of 4: code that aligned operands never run is
+        // kept small.
+        constexpr int UB = NP < 4 ? NP : 4;
+        const uint16_t* col = reinterpret_cast<const uint16_t*>(optr) + n0 + 8 * cchk;
+        const int n = n0 + 8 * cchk;
+#pragma clang loop unroll(disable)
+        for (int b = 0; b < NP / UB; ++b) {
+          i32x4_t x[UB];
+          static_for<0, UB>([&](auto q) {
+            const int m = m0 + (b * UB + q) * RPP + crow;
+            x[q] = i32x4_t{0, 0, 0, 0};
+            if (m < M && n + 8 <= N) x[q] = *reinterpret_cast<const i32x4_any_t*>(col + (int64_t)m * osm);
+          });
+          if (n < N && n + 8 > N) {
+            static_for<0, UB>([&](auto q) {
+              const int m = m0 + (b * UB + q) * RPP + crow;
+              if (m < M) x[q] = load_row_end(reinterpret_cast<const uint16_t*>(optr) + (int64_t)m * osm, n, N);
+            });
+          }
+          static_for<0, UB>([&](auto q) {
+            const int rl = (b * UB + q) * RPP + crow;
+            *reinterpret_cast<i32x4_t*>(stg + stage_chunk<BN>(rl, cchk)) =
+                stage_swapped<BN>(rl) ? swap_halves(x[q]) : x[q];
+          });
+        }
+      }
     }
     if (staged >= 0 && !op_dma) __syncthreads();
 
@@ -1176,12 +1326,17 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
     // vector's values (which depend only on the column) are read from LDS once
     // per column block.  Carrying one column block (not all of them) through the
     // runtime op loop keeps the loop's live values within the register file.
-    const bool use_stage_out = d.out.ptr != nullptr && (d.out.reserved & kFlagStage) && !col_red;
+    const bool use_stage_out = d.out.ptr != nullptr && (d.out.reserved & kFlagStage);
     // Activations run a step at a time across EW values (independent VALU
     // chains).  16 instead of 8 for the one-wave schedule measured no faster.
     constexpr int EW = 8;
     const bool out_bf16 = d.out.dtype == FUSEML_BF16;
     float rs[NJ], rmx[NJ];  // row partials (sum, max) of this lane's rows
+    float cls[NI], clm[NI];  // column partials: of one column per column block (below)
+    static_for<0, NI>([&](auto q) {
+      cls[q] = 0.0f;
+      clm[q] = -INFINITY;
+    });
     static_for<0, NJ>([&](auto j) {
       rs[j] = 0.0f;
       rmx[j] = -INFINITY;
@@ -1363,12 +1518,8 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
               run([](uint32_t h) { return f16_bits_to_f32(h); });
           } else {
             static_for<0, NJ>([&](auto j) {
-              const int m = mw + 32 * j;
               float x[16];
-              static_for<0, 4>([&](auto g) {
-                const int n = nb + 8 * g;
-                load_operand4(d.operands[oi], m0, n0, m, n, m < M && n < N, x + 4 * g);
-              });
+              load_operand16(d.operands[oi], m0, n0, mw + 32 * j, nb, M, N, x);
               combine(A[j], x);
             });
           }
@@ -1376,13 +1527,7 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
         }
         switch (kind) {
           case FUSEML_OP_STORE:
-            static_for<0, NJ>([&](auto j) {
-              static_for<0, 4>([&](auto g) {
-                const float x[4] = {A[j][4 * g], A[j][4 * g + 1], A[j][4 * g + 2],
-                                    A[j][4 * g + 3]};
-                store_out4(d.extra[oi], mw + 32 * j, nb + 8 * g, M, N, x);
-              });
-            });
+            static_for<0, NJ>([&](auto j) { store_out16(d.extra[oi], mw + 32 * j, nb, M, N, A[j]); });
             break;
 #define FUSEML_EACH(expr)                                \
   static_for<0, NJ>([&](auto j) {                        \
@@ -1436,11 +1581,6 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
       // values stay in registers from the first op to the LDS write.  The staged
       // output overwrites the staged operand in place: each 8-byte unit is read
       // (above) and written (here) by the same lane.
-      float cs[16], cmx[16];
-      static_for<0, 16>([&](auto r) {
-        cs[r] = 0.0f;
-        cmx[r] = -INFINITY;
-      });
       // Coordinates from an opaque lane copy, as in the op loop: derived from
       // the tile-wide ones, their 64-bit forms are hoisted and held (spilled).
       int ln = lane;
@@ -1478,14 +1618,7 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
           asm volatile("; staged output block, fp16");
         }
       } else if (d.out.ptr != nullptr) {
-        static_for<0, NJ>([&](auto j) {
-          const int m = mw + 32 * j;
-          const int nb = nw + 32 * i;
-          static_for<0, 4>([&](auto g) {
-            const float x[4] = {A[j][4 * g], A[j][4 * g + 1], A[j][4 * g + 2], A[j][4 * g + 3]};
-            store_out4(d.out, m, nb + 8 * g, M, N, x);
-          });
-        });
+        static_for<0, NJ>([&](auto j) { store_out16(d.out, mw + 32 * j, nw + 32 * i, M, N, A[j]); });
       }
       // Partial reductions exclude every element outside [0,M) x [0,N) (the
       // reference lets padded tile elements through, kernel_generator.py:1959-1960,
@@ -1511,42 +1644,62 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
             rs[j] += s8[0] + s8[1];
             rmx[j] = max_nan(rmx[j], max_nan(m8[0], m8[1]));
           });
-        } else if (row_red || col_red) {
+        } else if (row_red) {
           static_for<0, NJ>([&](auto j) {
             const int m = mw + 32 * j;
             const int nb = nw + 32 * i;
             static_for<0, 16>([&](auto r) {
               const int n = nb + 8 * (r >> 2) + (r & 3);
-              const bool in = (m < M) && (n < N);
               const float x = A[j][(int)r];
-              if (row_red && in) {
+              if (m < M && n < N) {
                 rs[j] += x;
                 rmx[j] = max_nan(rmx[j], x);
               }
-              if (col_red && in) {
-                cs[r] += x;
-                cmx[r] = max_nan(cmx[r], x);
-              }
             });
           });
+        } else if (col_red) {
+          // Column partials: first over this lane's row blocks, then over the 32
+          // rows of its half-wave by halving: at lane distance 16, 8, 4 and 2 a
+          // lane hands over the half of its columns that its partner keeps, so 16
+          // exchanges (and one more at distance 1) leave every lane with the sum
+          // of one column, r = (l32 >> 1), where a full exchange of each column
+          // takes 80.  The 16x fewer values stay in registers until the output
+          // is drained, so the output and a 2-D operand are staged in LDS as they
+          // are beside row reductions (16384x4096x1024 ReLU + three column
+          // reductions, bf16: 227.7 -> 165.1 us; over rows 137.0).
+          float cs[16], cmx[16];
+          static_for<0, 16>([&](auto r) {
+            const int n = nw + 32 * i + 8 * (r >> 2) + (r & 3);
+            cs[r] = 0.0f;
+            cmx[r] = -INFINITY;
+            static_for<0, NJ>([&](auto j) {
+              const float x = A[j][(int)r];
+              const bool in = interior || (mw + 32 * j < M && n < N);
+              cs[r] += in ? x : 0.0f;
+              cmx[r] = max_nan(cmx[r], in ? x : -INFINITY);
+            });
+          });
+          auto halve = [&](auto dist) {
+            constexpr int DIST = decltype(dist)::value, H = DIST / 2;
+            const bool up = (l32 & DIST) != 0;
+            static_for<0, H>([&](auto q) {
+              const float so = up ? cs[q] : cs[q + H], sk = up ? cs[q + H] : cs[q];
+              const float mo = up ? cmx[q] : cmx[q + H], mk = up ? cmx[q + H] : cmx[q];
+              cs[q] = sk + lane_xor<DIST>(so);
+              cmx[q] = max_nan(mk, lane_xor<DIST>(mo));
+            });
+          };
+          halve(std::integral_constant<int, 16>{});
+          halve(std::integral_constant<int, 8>{});
+          halve(std::integral_constant<int, 4>{});
+          halve(std::integral_constant<int, 2>{});
+          cs[0] += lane_xor<1>(cs[0]);
+          cmx[0] = max_nan(cmx[0], lane_xor<1>(cmx[0]));
+          static_for<0, NI>([&](auto q) {
+            cls[q] = i == q ? cs[0] : cls[q];
+            clm[q] = i == q ? cmx[0] : clm[q];
+          });
         }
-      }
-      if (RED && col_red) {
-        // Column partials: reduce over the 32 rows held by each half-wave.  Column
-        // reductions use neither a staged output nor a staged operand (the host
-        // does not flag them), so the staging tile's LDS is free here.
-        static_for<0, 16>([&](auto r) {
-  #pragma unroll
-          for (int sh = 1; sh < 32; sh <<= 1) {
-            cs[r] += __shfl_xor(cs[r], sh);
-            cmx[r] = max_nan(cmx[r], __shfl_xor(cmx[r], sh));
-          }
-          if (l32 == 0) {
-            const int col = wn * TN + 32 * i + 8 * (r >> 2) + 4 * khalf + (r & 3);
-            red_sum[wm * BN + col] = cs[r];
-            red_max[wm * BN + col] = cmx[r];
-          }
-        });
       }
     };
     if constexpr (SCHED >= 3) {
@@ -1605,24 +1758,51 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
       // 16 passes unrolled: their LDS reads are in flight together (measured 2%
       // faster than 4 at 16384x4096x1024 with no ops; the kernel's code is small
       // enough since the column blocks share one copy of the op code).
+      if (d.out.reserved & kFlagAligned) {
 #pragma unroll 16
-      for (int p = 0; p < BM / RPP; ++p) {
-        const int rl = p * RPP + crow;
-        const int m = m0 + rl, n = n0 + 8 * cchk;
-        i32x4_t x = *reinterpret_cast<const i32x4_t*>(stg + stage_chunk<BN>(rl, cchk));
-        if (stage_swapped<BN>(rl)) x = swap_halves(x);
-        if (m < M && n < N) {
+        for (int p = 0; p < BM / RPP; ++p) {
+          const int rl = p * RPP + crow;
+          const int m = m0 + rl, n = n0 + 8 * cchk;
+          i32x4_t x = *reinterpret_cast<const i32x4_t*>(stg + stage_chunk<BN>(rl, cchk));
+          if (stage_swapped<BN>(rl)) x = swap_halves(x);
+          if (m < M && n < N) {
+            uint16_t* dst = reinterpret_cast<uint16_t*>(d.out.ptr) + (int64_t)m * d.out.ld + n;
+            *reinterpret_cast<i32x4_t*>(dst) = x;
+          }
+        }
+      } else {
+#pragma unroll 4
+        for (int p = 0; p < BM / RPP; ++p) {
+          const int rl = p * RPP + crow;
+          const int m = m0 + rl, n = n0 + 8 * cchk;
+          i32x4_t x = *reinterpret_cast<const i32x4_t*>(stg + stage_chunk<BN>(rl, cchk));
+          if (stage_swapped<BN>(rl)) x = swap_halves(x);
           uint16_t* dst = reinterpret_cast<uint16_t*>(d.out.ptr) + (int64_t)m * d.out.ld + n;
-          *reinterpret_cast<i32x4_t*>(dst) = x;
+          if (m < M && n + 8 <= N) *reinterpret_cast<i32x4_any_t*>(dst) = x;
+        }
+      }
+      // Row ends that are no whole chunk, in the tile that holds them: element
+      // by element, a row per thread.
+      if ((N & 7) != 0 && n0 + BN > N) {
+        const int ce = (N - n0) >> 3;
+        for (int rl = tid; rl < BM; rl += NT) {
+          const int m = m0 + rl;
+          if (m >= M) break;
+          i32x4_t x = *reinterpret_cast<const i32x4_t*>(stg + stage_chunk<BN>(rl, ce));
+          if (stage_swapped<BN>(rl)) x = swap_halves(x);
+          uint16_t* dst = reinterpret_cast<uint16_t*>(d.out.ptr) + (int64_t)m * d.out.ld + n0 + 8 * ce;
+          static_for<0, 7>([&](auto e) {
+            if (e < (N & 7)) dst[e] = (uint16_t)((uint32_t)x[(int)(e / 2)] >> (16 * (e & 1)));
+          });
         }
       }
     }
 
     if (!RED || d.reduce_mask == 0) continue;
+    // The partials overwrite the staging tile, which other waves may still be
+    // draining (staged output) or reading (staged operand).
+    if (use_stage_out || staged >= 0) lds_barrier();
     if (row_red) {
-      // The partials overwrite the staging tile, which other waves may still be
-      // draining (staged output) or reading (staged operand).
-      if (use_stage_out || staged >= 0) lds_barrier();
       // Row partials: the other half-wave holds the other 4-column runs of the same rows.
       static_for<0, NJ>([&](auto j) {
         const float s2 = rs[j] + __shfl_xor(rs[j], 32);
@@ -1632,6 +1812,14 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
           red_sum[wn * BM + row] = s2;
           red_max[wn * BM + row] = m2;
         }
+      });
+    } else if ((lane & 1) == 0) {
+      // Column partials (halve(), above): column r = l32 / 2 of each column block.
+      const int r = l32 >> 1;
+      static_for<0, NI>([&](auto q) {
+        const int col = wn * TN + 32 * q + 8 * (r >> 2) + 4 * khalf + (r & 3);
+        red_sum[wm * BN + col] = cls[q];
+        red_max[wm * BN + col] = clm[q];
       });
     }
     lds_barrier();

@@ -15,7 +15,8 @@ namespace fuseml_gemm {
 
 // Host-derived flags kept in the `reserved` field of operands and outputs.
 constexpr int kFlagVec4 = 1;   // unit stride along N, rows 4-element aligned: 8/16-byte vectors
-constexpr int kFlagStage = 2;  // 16-bit, rows 8-element aligned, 16-byte base: LDS-staged tile
+constexpr int kFlagStage = 2;  // 16-bit, unit stride along N, N >= 8: LDS-staged tile
+constexpr int kFlagAligned = 8;  // a staged tile's rows are whole 16-byte chunks at 16-byte addresses
 constexpr int kFlagAux = 4;    // row ([N]) or column ([M]) vector staged as fp32 in LDS slot (bits 8-9)
 constexpr int kAuxSlots = 4;   // vector operands staged per launch
 
