@@ -160,12 +160,13 @@ TileConfig choose_config(const fuseml_gemm_desc& d, int cus) {
   // K = 1024, on full rounds and on a partial one (136 to 224 tiles) alike: bf16
   // ReLU, residual and act-heavy chains 0.94-1.01 of the ping-pong kernel's time
   // at K = 1024 and 0.91-0.96 at K = 4096, fp16 ones 0.92-1.00 and 0.89-0.95
-  // (8192x4096x4096 bias+residual, fp16, 260 -> 231 us).  bias+GELU(erf), the
-  // chain with the most VALU work, only from K = 2048 (0.94-1.02 there, 0.92-0.97
-  // at K = 4096; 1.00-1.05 at K = 1024).  Its generic op loop loses 3-17% below
-  // K = 2048 and on partial rounds, and wins from K = 2048 with at least one
-  // full round of tiles or from K = 8192.  With K % 64 != 0 the two-stage one
-  // takes over from K = 8192.
+  // (8192x4096x4096 bias+residual, fp16, 260 -> 231 us).  The GELU(erf) chains,
+  // those with the most VALU work, only from K = 2048 (0.94-1.02 there, 0.92-0.97
+  // at K = 4096; 1.00-1.06 at K = 1024), or with 7/8 of a round from K = 1536
+  // (0.95-0.99) and fp16 from K = 1024 (0.98-1.00).  Its generic op loop loses
+  // 3-17% below K = 2048 and below 224 tiles, and wins from K = 2048 with at
+  // least 7/8 of a round (0.94-1.00 at 224 tiles) or from K = 8192.  With K % 64
+  // != 0 the two-stage one takes over from K = 8192.
   // Below one round of 256x256 tiles (2 x large_tiles <= cus) the smaller
   // tiles (choose_partial_round): at 128 large tiles on 256 CUs the 128x128
   // one was 7-17% faster than 256x256 (bias+GELU at K = 512-1024), from 144
@@ -180,10 +181,12 @@ TileConfig choose_config(const fuseml_gemm_desc& d, int cus) {
   if (weight_streaming(d, cus)) return d.M <= 32 ? kNarrow32 : d.M <= 64 ? kNarrow64 : kSmall64;
   const int64_t large_tiles = cdiv(d.M, 256) * cdiv(d.N, 256);
   if (2 * large_tiles <= cus || d.M <= 128) return choose_partial_round(d, cus);
-  if (d.K % 64 == 0 && (d.K >= 8192 || (d.K >= 2048 && large_tiles >= cus))) return kDeep3;
+  if (d.K % 64 == 0 && (d.K >= 8192 || (d.K >= 2048 && 8 * large_tiles >= 7 * cus))) return kDeep3;
   if (d.K % 64 == 0 && d.K >= 1024) {
     const int ch = match_fixed_chain(d);
-    if (ch != kChainGeneric && (ch != kChainBiasGeluErf || d.K >= 2048)) return kDeep3;
+    const bool gelu = ch == kChainBiasGeluErf || ch == kChainBiasGeluScale;
+    const int64_t gelu_k = 8 * large_tiles < 7 * cus ? 2048 : d.ab_dtype == FUSEML_F16 ? 1024 : 1536;
+    if (ch != kChainGeneric && (!gelu || d.K >= gelu_k)) return kDeep3;
   }
   return d.K >= 8192 ? kDeep : kLarge;
 }
@@ -457,6 +460,10 @@ int match_fixed_chain(const fuseml_gemm_desc& d) {
       else if (row(0) && is(1, FUSEML_OP_RELU)) ch = kChainBiasRelu;
       else if (row(0) && tile(1, FUSEML_OP_ADD)) ch = kChainBiasTile;
       break;
+    case 4:
+      if (row(0) && is(1, FUSEML_OP_GELU_ERF) && is(2, FUSEML_OP_SCALE) && is(3, FUSEML_OP_ADD_SCALAR))
+        ch = kChainBiasGeluScale;
+      break;
     case 5:
       if (row(0) && is(1, FUSEML_OP_RELU) && tile(2, FUSEML_OP_MUL) && is(3, FUSEML_OP_SIGMOID) && row(4))
         ch = kChainActHeavy;
@@ -520,6 +527,7 @@ hipError_t launch_fixed(const fuseml_gemm_desc& d, int ch, hipStream_t stream, i
     case kChainBiasTile: launch_fixed_one<C, T, kChainBiasTile>(d, stream, grid, block); break;
     case kChainActHeavy: launch_fixed_one<C, T, kChainActHeavy>(d, stream, grid, block); break;
     case kChainRelu: launch_fixed_one<C, T, kChainRelu>(d, stream, grid, block); break;
+    case kChainBiasGeluScale: launch_fixed_one<C, T, kChainBiasGeluScale>(d, stream, grid, block); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -556,6 +564,87 @@ int device_cus(int dev) {
   }
   if (dev >= 0 && dev < kMaxDevices) g_device_cus[dev].store(cus, std::memory_order_relaxed);
   return cus;
+}
+
+// One launch of `d` (flags derived) on the kernel its size and chain choose.
+hipError_t launch_one(const fuseml_gemm_desc& d, int cus, hipStream_t stream) {
+  const int ks = choose_ksplit(d, cus);
+  if (ks >= 0)
+    return d.ab_dtype == FUSEML_BF16 ? launch_ksplit<__bf16>(d, ks, stream) : launch_ksplit<_Float16>(d, ks, stream);
+  const TileConfig c = choose_config(d, cus);
+  const int ch = launch_chain(d, c);
+  if (ch != kChainGeneric)
+    return d.ab_dtype == FUSEML_BF16 ? launch_fixed<kDeep3, __bf16>(d, ch, stream, cus)
+                                     : launch_fixed<kDeep3, _Float16>(d, ch, stream, cus);
+  if (c.sched == kDeep.sched) return launch_variant<kDeep>(d, stream, cus);
+  if (c.sched == kLarge.sched && c.bn == kLarge128.bn) return launch_variant<kLarge128>(d, stream, cus);
+  if (c.sched == kLarge.sched) return launch_variant<kLarge>(d, stream, cus);
+  if (c.sched == kDeep3.sched) return launch_variant<kDeep3>(d, stream, cus);
+  if (c.bm == kSmall64.bm && c.bk == kSmall64.bk) return launch_variant<kSmall64>(d, stream, 0);
+  if (c.bm == kNarrow64.bm) return launch_variant<kNarrow64>(d, stream, 0);
+  if (c.bm == kNarrow32.bm) return launch_variant<kNarrow32>(d, stream, 0);
+  return launch_variant<kSmall>(d, stream, 0);
+}
+
+// The rows from m1 on (or the columns from n1 on) of `d` as a group of their own.
+fuseml_gemm_desc rest_of(const fuseml_gemm_desc& d, int64_t m1, int64_t n1) {
+  fuseml_gemm_desc r = d;
+  auto advance = [](const void* p, int64_t elements, int dtype) -> void* {
+    return p == nullptr ? nullptr : (char*)p + elements * (dtype == FUSEML_F32 ? 4 : 2);
+  };
+  r.M -= m1;
+  r.N -= n1;
+  r.a = advance(d.a, m1 * d.lda, d.ab_dtype);
+  r.b = advance(d.b, n1 * d.ldb, d.ab_dtype);
+  for (int i = 0; i < d.n_operands; ++i) {
+    fuseml_operand& o = r.operands[i];
+    const int64_t skip = m1 * o.stride_m + n1 * o.stride_n;
+    o.ptr = advance(o.ptr, skip, o.dtype);
+    o.extent -= skip;
+  }
+  r.out.ptr = advance(d.out.ptr, m1 * d.out.ld + n1, d.out.dtype);
+  for (int i = 0; i < d.n_extra; ++i)
+    r.extra[i].ptr = advance(d.extra[i].ptr, m1 * d.extra[i].ld + n1, d.extra[i].dtype);
+  if (d.reduce_mask != 0)
+    for (int b = 0; b < 3; ++b)
+      if (d.reduce_out[b] != nullptr) r.reduce_out[b] += d.reduce_axis == 1 ? m1 : n1;
+  return r;
+}
+
+// A last round of few 256x256 tiles takes nearly as long as a full one (a CU's
+// time for one tile: 23 us at K = 1024 and 67 at K = 4096 behind a full round, for
+// 16 to 64 tiles of 256), so it runs as a group of its own on the tiles of its
+// size: `d` keeps the whole rounds, `rest` the remaining rows (or columns, where
+// rows would leave more than 7% of the rounds idle).  Priced as choose_ksplit
+// prices a small group, 2 us for the second launch, and only where that is 0.9 of
+// the partial round or less.  Not for a mean along the split axis, whose divisor
+// is the whole length.  Measured (M x N x K, us, one launch -> two): see below.
+bool split_rounds(fuseml_gemm_desc& d, int cus, fuseml_gemm_desc& rest) {
+  if (forced_variant() != 0 || d.K <= 0 || d.M <= 128) return false;
+  const int64_t tm = cdiv(d.M, 256), tn = cdiv(d.N, 256), rounds = tm * tn / cus;
+  if (rounds == 0 || tm * tn % cus == 0) return false;
+  const int64_t m_tiles = rounds * cus / tn, n_tiles = rounds * cus / tm;
+  const bool by_rows = m_tiles * tn >= n_tiles * tm;
+  const int64_t kept = by_rows ? m_tiles * tn : n_tiles * tm;
+  if (kept * 100 < rounds * cus * 93) return false;
+  if ((d.reduce_mask & FUSEML_RED_MEAN) && d.reduce_axis == (by_rows ? 0 : 1)) return false;
+  fuseml_gemm_desc r = rest_of(d, by_rows ? m_tiles * 256 : 0, by_rows ? 0 : n_tiles * 256);
+  if (2 * cdiv(r.M, 256) * cdiv(r.N, 256) > cus) return false;
+  const double k = (double)d.K / 1024.0;
+  const double left = (double)(tm * tn - rounds * cus) / cus;
+  const double partial = (8.3 + 14.7 * k) * (left > 0.25 ? 0.875 + 0.5 * left : 1.0);
+  double small = 0.0;
+  int64_t work = 0;
+  choose_partial_round(r, cus, &work);
+  cheapest_ksplit(r, cus, 0.32, &small);
+  const double tiled = -3.0 + (double)work / (5.0 * 160.0) * (5.05 + 3.6 * k);
+  if (small >= 0.85 * tiled) small = tiled;
+  if (small + 2.0 > 0.9 * partial) return false;
+  derive_flags(r);
+  rest = r;
+  if (by_rows) d.M = m_tiles * 256; else d.N = n_tiles * 256;
+  derive_flags(d);
+  return true;
 }
 
 }  // namespace
@@ -743,36 +832,14 @@ int fuseml_gemm_epilogue(const fuseml_gemm_desc* desc, void* stream_ptr) {
   if (rc != FUSEML_OK) return rc;
   hipError_t e = hipSuccess;
 
-  const int ks = choose_ksplit(d, cus);
-  if (ks >= 0) {
-    e = d.ab_dtype == FUSEML_BF16 ? launch_ksplit<__bf16>(d, ks, stream) : launch_ksplit<_Float16>(d, ks, stream);
-    if (e != hipSuccess) {
-      set_error("gemm_ksplit launch: %s", hipGetErrorString(e));
-      return FUSEML_EHIP;
-    }
-    return FUSEML_OK;
+  // The part of whole rounds, then the rest, each on the kernel of its own size.
+  fuseml_gemm_desc rest;
+  if (split_rounds(d, cus, rest)) {
+    e = launch_one(d, cus, stream);
+    if (e == hipSuccess) e = launch_one(rest, cus, stream);
+  } else {
+    e = launch_one(d, cus, stream);
   }
-  const TileConfig c = choose_config(d, cus);
-  const int ch = launch_chain(d, c);
-  if (ch != kChainGeneric)
-    e = d.ab_dtype == FUSEML_BF16 ? launch_fixed<kDeep3, __bf16>(d, ch, stream, cus)
-                                  : launch_fixed<kDeep3, _Float16>(d, ch, stream, cus);
-  else if (c.sched == kDeep.sched)
-    e = launch_variant<kDeep>(d, stream, cus);
-  else if (c.sched == kLarge.sched && c.bn == kLarge128.bn)
-    e = launch_variant<kLarge128>(d, stream, cus);
-  else if (c.sched == kLarge.sched)
-    e = launch_variant<kLarge>(d, stream, cus);
-  else if (c.sched == kDeep3.sched)
-    e = launch_variant<kDeep3>(d, stream, cus);
-  else if (c.bm == kSmall64.bm && c.bk == kSmall64.bk)
-    e = launch_variant<kSmall64>(d, stream, 0);
-  else if (c.bm == kNarrow64.bm)
-    e = launch_variant<kNarrow64>(d, stream, 0);
-  else if (c.bm == kNarrow32.bm)
-    e = launch_variant<kNarrow32>(d, stream, 0);
-  else
-    e = launch_variant<kSmall>(d, stream, 0);
   if (e != hipSuccess) {
     set_error("gemm_epilogue launch: %s", hipGetErrorString(e));
     return FUSEML_EHIP;

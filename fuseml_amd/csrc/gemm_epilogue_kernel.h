@@ -1348,12 +1348,18 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
     // the row-vector ADD of every chain that has one; the act-heavy chain's
     // second row vector is op 4, and the tile ADD of bias + tile is op 1.
     constexpr bool kFxRow0 = CH == kChainBias || CH == kChainBiasGeluErf || CH == kChainBiasGeluTanh ||
-                             CH == kChainBiasRelu || CH == kChainBiasTile || CH == kChainActHeavy;
+                             CH == kChainBiasRelu || CH == kChainBiasTile || CH == kChainActHeavy ||
+                             CH == kChainBiasGeluScale;
     int fx_slot0 = 0, fx_slot1 = 0;
     float fx_a0 = 1.0f, fx_a1 = 1.0f;
     if constexpr (kFxRow0) {
       fx_slot0 = (d.operands[d.ops[0].operand].reserved >> 8) & (kAuxSlots - 1);
       fx_a0 = d.ops[0].scalar;
+    }
+    float fx_s0 = 1.0f, fx_s1 = 0.0f;
+    if constexpr (CH == kChainBiasGeluScale) {
+      fx_s0 = d.ops[2].scalar;
+      fx_s1 = d.ops[3].scalar;
     }
     if constexpr (CH == kChainBiasTile) fx_a1 = d.ops[1].scalar;
     if constexpr (CH == kChainActHeavy) {
@@ -1415,7 +1421,17 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
         });
       };
       if constexpr (kFxRow0) add_row(fx_slot0, fx_a0);
-      if constexpr (CH == kChainBiasGeluErf) activation([](float* v) { gelu_erf_n<16>(v); });
+      if constexpr (CH == kChainBiasGeluErf || CH == kChainBiasGeluScale) activation([](float* v) { gelu_erf_n<16>(v); });
+      if constexpr (CH == kChainBiasGeluScale) {
+        // Two rounded steps, as the op loop takes them (one FMA would round once).
+        static_for<0, NJ>([&](auto j) {
+          static_for<0, 16>([&](auto r) {
+#pragma clang fp contract(off)
+            const float scaled = A[j][(int)r] * fx_s0;
+            A[j][(int)r] = scaled + fx_s1;
+          });
+        });
+      }
       if constexpr (CH == kChainBiasGeluTanh) activation([](float* v) { gelu_tanh_n<16>(v); });
       if constexpr (CH == kChainBiasRelu || CH == kChainRelu || CH == kChainActHeavy) relu_all();
       if constexpr (CH == kChainBiasTile || CH == kChainActHeavy) {

@@ -74,7 +74,8 @@ enum FixedChain : int {
   kChainBiasTile = 6,      // add(row), add(tile)           (bias + residual)
   kChainActHeavy = 7,      // add(row), relu, mul(tile), sigmoid, add(row)
   kChainRelu = 8,          // relu                          (also with reductions)
-  kNumChains = 9,
+  kChainBiasGeluScale = 9,  // add(row), gelu(approximate='none'), scale, add_scalar
+  kNumChains = 10,
 };
 
 // The kernel (defined in gemm_epilogue_kernel.h).  SCHED selects the K-loop

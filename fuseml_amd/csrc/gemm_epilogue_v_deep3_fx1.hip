@@ -6,3 +6,4 @@
 
 FUSEML_GEMM_INSTANTIATE_ONE(fuseml_gemm::kDeep3, __bf16, false, fuseml_gemm::kChainBiasGeluErf)
 FUSEML_GEMM_INSTANTIATE_ONE(fuseml_gemm::kDeep3, __bf16, false, fuseml_gemm::kChainBiasGeluTanh)
+FUSEML_GEMM_INSTANTIATE_ONE(fuseml_gemm::kDeep3, __bf16, false, fuseml_gemm::kChainBiasGeluScale)

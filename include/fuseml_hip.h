@@ -182,7 +182,7 @@ int fuseml_gemm_epilogue_f32_supported(const fuseml_gemm_desc* desc);
  * (the descriptor's ops interpreted at run time), else the id of the fixed
  * chain kernel (1 none, 2 bias, 3 bias+GELU(erf), 4 bias+GELU(tanh),
  * 5 bias+ReLU, 6 bias+2-D add, 7 bias,ReLU,2-D mul,sigmoid,row add, 8 ReLU
- * with or without reductions) — the same arithmetic as straight-line code,
+ * with or without reductions, 9 bias+GELU(erf), scale, scalar add) — the same arithmetic as straight-line code,
  * built for the one-wave whole-stage variant and GEMM operands of one type with
  * the output where they are fp16.  A negative
  * FUSEML_E* code for an invalid descriptor.  For tests and measurement; it

@@ -48,6 +48,21 @@ def test_fp16_fixed_chain_bitwise_equals_generic(name, shape):
     _check_tile(fixed, ref, f"fp16 fixed {name} {shape}")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("shape", [(600, 1032, 192), (4392, 4360, 128)], ids=lambda s: "x".join(map(str, s)))
+def test_gelu_scale_fixed_chain_bitwise_equals_generic(shape, dtype):
+    """The activation-heavy block's first group: GELU, then a scale and a scalar
+    add, each rounded."""
+    M, N, K = shape
+    a, w = _gemm_inputs(M, N, K, dtype, seed=96)
+    host = [_operands(M, N, dtype, seed=97)[0], a, w.t()]
+    steps = [("add", 0, 1.0), ("gelu_erf", -1, 1.0), ("scale", -1, 0.3), ("add_scalar", -1, 0.125)]
+    spec = _spec(left=1, right=2, ops=steps, out_dtype=dtype)
+    fixed, generic = _both(spec, [t.cuda() for t in host], 9)
+    assert torch.equal(fixed, generic)
+    _check_tile(fixed, ora.gemm_epilogue([_np(t) for t in host], 1, 2, steps)["tile"])
+
+
 @pytest.mark.parametrize("axis", [1, 0])
 def test_fp16_fixed_relu_reductions_equal_generic(axis):
     dtype = torch.float16
