@@ -265,6 +265,16 @@ def load_library() -> ctypes.CDLL:
         return lib
 
 
+def load_fastcall():
+    """The launchers' native-call extension; ImportError if it is not built."""
+    try:
+        from . import _fastcall
+    except ImportError as exc:
+        raise ImportError(f"fuseml_amd/_fastcall.so cannot be loaded ({exc}) — run `python -m fuseml_amd.build` "
+                          "(or __graft_entry__.build()) first") from exc
+    return _fastcall
+
+
 VARIANTS = ("large", "deep", "deep3", "small", "narrow64", "narrow32", "large128", "small64")
 
 

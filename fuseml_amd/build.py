@@ -1,9 +1,10 @@
-"""Build the gfx950 HIP kernel library in-tree: ``python -m fuseml_amd.build``.
+"""Build the native parts in-tree: ``python -m fuseml_amd.build``.
 
 Each ``fuseml_amd/csrc/*.hip`` is compiled by its own ``hipcc -c`` for
 ``--offload-arch=gfx950`` only (in parallel: the GEMM kernels are split one
 tile variant per translation unit), and the objects are linked into
-``fuseml_amd/libfuseml_hip.so``.  The build is ahead-of-time: there is no
+``fuseml_amd/libfuseml_hip.so``; ``csrc/fastcall.cpp`` (the launchers' native
+calls, no GPU code) becomes ``fuseml_amd/_fastcall.so``.  The build is ahead-of-time: there is no
 runtime JIT (the reference compiles Triton kernels on the first call,
 fuseml/codegen/kernel_generator.py:1067-1172).
 """
@@ -22,6 +23,7 @@ REPO_DIR = os.path.dirname(PKG_DIR)
 INCLUDE_DIR = os.path.join(REPO_DIR, "include")
 CSRC_DIR = os.path.join(PKG_DIR, "csrc")
 LIB_PATH = os.path.join(PKG_DIR, "libfuseml_hip.so")
+FASTCALL_PATH = os.path.join(PKG_DIR, "_fastcall.so")
 OBJ_DIR = os.path.join(PKG_DIR, "_build")
 
 ARCH = "gfx950"
@@ -60,6 +62,21 @@ def _run(cmd: list[str], verbose: bool) -> None:
         print(err, file=sys.stderr)
 
 
+def fastcall_command(out: str) -> list[str]:
+    """The host compiler's line for the CPython extension of the launchers."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    return [os.environ.get("CXX") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{INCLUDE_DIR}",
+            *[a for p in include_paths() for a in ("-isystem", p)], f"-I{sysconfig.get_paths()['include']}",
+            os.path.join(CSRC_DIR, "fastcall.cpp"), "-o", out, f"-L{lib}", "-ltorch_python", "-ltorch", "-ltorch_cpu",
+            "-lc10"]
+
+
 def build(verbose: bool = False, jobs: int | None = None) -> str:
     """Compile every HIP source and link the in-tree shared library; return its path."""
     srcs = sources()
@@ -68,7 +85,9 @@ def build(verbose: bool = False, jobs: int | None = None) -> str:
     os.makedirs(OBJ_DIR, exist_ok=True)
     cc = hipcc()
     objs = [os.path.join(OBJ_DIR, os.path.splitext(os.path.basename(s))[0] + ".o") for s in srcs]
+    fast_tmp = FASTCALL_PATH + ".tmp"
     cmds = [[cc, *HIPCC_FLAGS, f"-I{INCLUDE_DIR}", "-c", s, "-o", o] for s, o in zip(srcs, objs)]
+    cmds.append(fastcall_command(fast_tmp))
     workers = jobs or min(len(cmds), max(1, len(os.sched_getaffinity(0))), 16)
     with concurrent.futures.ThreadPoolExecutor(max_workers=workers) as pool:
         for f in [pool.submit(_run, c, verbose) for c in cmds]:
@@ -76,6 +95,7 @@ def build(verbose: bool = False, jobs: int | None = None) -> str:
     tmp = LIB_PATH + ".tmp"
     _run([cc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp], verbose)
     os.replace(tmp, LIB_PATH)
+    os.replace(fast_tmp, FASTCALL_PATH)
     return LIB_PATH
 
 

@@ -64,9 +64,9 @@ class EagerFallbackGuard:
         except Exception as exc:  # noqa: BLE001 - filtered below
             if not self.is_recoverable(exc):
                 raise
-            return self._fallback(exc, inputs)
+            return self.recover(exc, inputs)
 
-    def _fallback(self, exc: BaseException, inputs: Sequence[Any]) -> Any:
+    def recover(self, exc: BaseException, inputs: Sequence[Any]) -> Any:
         self._fallback_count += 1
         logger.warning(
             "fused kernel '%s' failed (#%d): %s: %s — running the eager path",

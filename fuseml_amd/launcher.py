@@ -124,7 +124,7 @@ class _Plan:
 
     __slots__ = ("desc", "M", "N", "K", "neg", "operands", "nbytes", "k_split", "fast", "words", "desc_ref",
                  "a_ok", "b_ok", "lda", "ldb", "op_words", "red_words", "extra_words", "single_tile", "direct",
-                 "split_plan")
+                 "split_plan", "native")
 
     def __init__(self) -> None:
         self.desc = _abi.GemmDesc()
@@ -146,6 +146,7 @@ class _Plan:
         self.single_tile = False
         self.direct = False
         self.split_plan: Optional["_Plan"] = None
+        self.native: Optional[bool] = None  # handed to the native caller; None: its signature was seen once
 
 
 class HipKernelLauncher:
@@ -168,7 +169,7 @@ class HipKernelLauncher:
             self._fallback_guard = EagerFallbackGuard(
                 eager_fn=eager_fn, kernel_signature=kernel_signature or spec.describe()
             )
-        self.launch_count = 0
+        self._python_launches = 0
         # Measurement hook: a list to receive, per launch, (start event, end
         # event, (M, N, K), algorithmic bytes) recorded on the launch stream
         # around the C call.  None (the default) records nothing.  Pairs of
@@ -178,8 +179,16 @@ class HipKernelLauncher:
         self.timing_pool: List[Tuple[Any, Any]] = []
         # Input slots the launch reads: the GEMM operands and the epilogue operands.
         self._used = sorted({spec.left, spec.right} | {op.operand for op in spec.ops if op.kind in ("add", "mul")})
+        # Later calls of a signature whose plan needs only pointers run in native
+        # code (csrc/fastcall.cpp); it declines every other call.
+        self._native = _abi.load_fastcall().Launcher(n_inputs, tuple(self._used), self._fallback_guard is not None)
+        self._native_call = self._native.call
 
     # ------------------------------------------------------------------
+    @property
+    def launch_count(self) -> int:
+        return self._python_launches + self._native.count
+
     @property
     def fallback_count(self) -> int:
         return self._fallback_guard.fallback_count if self._fallback_guard else 0
@@ -317,6 +326,11 @@ class HipKernelLauncher:
         if plan is None:
             plan = self._make_plan(inputs)
             self._plans[key] = plan
+        elif plan.native is None:
+            # The signature came back: its next calls run in native code.
+            plan.native = plan.fast and plan.a_ok and plan.b_ok and isinstance(self._lib, ctypes.CDLL)
+            if plan.native:
+                self._add_native(plan, inputs)
         if plan.direct and (inputs[self.spec.left].data_ptr() | inputs[self.spec.right].data_ptr()) % 16:
             if plan.split_plan is None:
                 plan.split_plan = self._make_plan(inputs, allow_direct=False)
@@ -326,6 +340,24 @@ class HipKernelLauncher:
         if plan.fast and self.timing_events is None and isinstance(self._lib, ctypes.CDLL):
             return self._launch_fast(plan, inputs)
         return self._launch_general(plan, inputs)
+
+    def _add_native(self, plan: _Plan, inputs: Sequence[torch.Tensor]) -> None:
+        """Hand a plan whose calls need only pointers to the native caller, unless
+        its results are cast or viewed after the launch."""
+        spec = self.spec
+        if spec.output_shapes or any(dt != torch.float32 for dt in spec.reduce_dtypes):
+            return
+        desc = _abi.GemmDesc()
+        ctypes.memmove(ctypes.byref(desc), plan.desc_ref, ctypes.sizeof(desc))
+        desc.lda, desc.ldb = plan.lda, plan.ldb
+        entry = self._lib.fuseml_gemm_epilogue_f32 if plan.direct else self._lib.fuseml_gemm_epilogue
+        names = list(spec.reductions)
+        outputs = tuple(("t", 0) if o[0] == "tile" else ("r", names.index(o[1])) if o[0] == "red" else ("e", o[1])
+                        for o in spec.outputs)
+        self._native.add(tuple(inputs), bytes(desc), ctypes.cast(entry, ctypes.c_void_p).value, spec.left, spec.right,
+                         tuple((slot, idx) for slot, (idx, _) in enumerate(plan.operands)),
+                         spec.out_dtype if spec.store_tile else None, tuple(spec.extra_dtypes),
+                         tuple(_abi.RED_SLOT[name] for name in names), outputs)
 
     def _launch_fast(self, plan: _Plan, inputs: Sequence[torch.Tensor]) -> Any:
         """A call whose plan needs only pointers: the same checks, allocations
@@ -380,7 +412,7 @@ class HipKernelLauncher:
         rc = entry(plan.desc_ref, torch._C._cuda_getCurrentRawStream(dev))
         if rc != _abi.OK:
             raise _abi.FuseMLHipError(rc, _abi.last_error(self._lib))
-        self.launch_count += 1
+        self._python_launches += 1
         if plan.single_tile:
             return tile
         return self._assemble(tile, extras, reds)
@@ -460,7 +492,7 @@ class HipKernelLauncher:
                 outs = [t for t in [tile, *extras, *reds.values()] if t is not None]
                 plan.nbytes = _distinct_bytes([inputs[i] for i in self._used] + outs)
             timing.append((ev0, ev1, (M, N, plan.K), plan.nbytes))
-        self.launch_count += 1
+        self._python_launches += 1
         return self._assemble(tile, extras, reds)
 
     def _split_operands(self, plan: _Plan, a: torch.Tensor, b: torch.Tensor, stream: int):
@@ -502,6 +534,18 @@ class HipKernelLauncher:
 
     # ------------------------------------------------------------------
     def __call__(self, *inputs: torch.Tensor) -> Any:
+        if self.timing_events is None:
+            try:
+                out = self._native_call(inputs)
+                if type(out) is int:
+                    raise _abi.FuseMLHipError(out, _abi.last_error(self._lib))
+            except Exception as exc:  # noqa: BLE001 - as the guard filters them
+                guard = self._fallback_guard
+                if guard is None or not guard.is_recoverable(exc):
+                    raise
+                return guard.recover(exc, inputs)
+            if out is not None:
+                return out
         if len(inputs) != self._n_inputs:
             raise ValueError(f"Expected {self._n_inputs} input tensor(s), got {len(inputs)}.")
         if self._fallback_guard is not None:
