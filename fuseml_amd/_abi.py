@@ -15,7 +15,7 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
-from typing import Optional
+from typing import Dict, Optional
 
 ABI_VERSION = 6
 MAX_OPS = 16
@@ -263,6 +263,19 @@ def load_library() -> ctypes.CDLL:
         _declare(lib)
         _lib = lib
         return lib
+
+
+_entries: Dict[bool, int] = {}
+
+
+def entry_address(f32: bool) -> int:
+    """The address of fuseml_gemm_epilogue (or of its fp32-operand form) in the
+    loaded library, for the native caller."""
+    if not _entries:
+        lib = load_library()
+        for key, fn in ((False, lib.fuseml_gemm_epilogue), (True, lib.fuseml_gemm_epilogue_f32)):
+            _entries[key] = ctypes.cast(fn, ctypes.c_void_p).value
+    return _entries[f32]
 
 
 def load_fastcall():

@@ -194,21 +194,24 @@ PyObject* launcher_call(PyObject* self_, PyObject* inputs) {
 }
 
 // add(inputs, desc, entry, left, right, operands, tile, extras, reductions, outputs):
-// a plan for the signature of `inputs`.  `desc`: the descriptor's bytes, `entry`:
+// a plan for the signature of `inputs`.  `desc`: the descriptor (a buffer), `entry`:
 // the C function's address, `tile`: the output's dtype or None, `extras`: dtypes,
 // the rest as in Plan.  Whether the plan was taken.
 PyObject* launcher_add(PyObject* self_, PyObject* args) {
   HANDLE_TH_ERRORS
   Launcher* self = reinterpret_cast<Launcher*>(self_);
   PyObject *inputs, *operands, *tile, *extras, *reductions, *outputs;
-  const char* desc;
-  Py_ssize_t desc_len;
+  Py_buffer desc;
   unsigned long long entry;
   int left, right;
-  if (!PyArg_ParseTuple(args, "O!y#KiiO!OO!O!O!", &PyTuple_Type, &inputs, &desc, &desc_len, &entry, &left, &right,
-                        &PyTuple_Type, &operands, &tile, &PyTuple_Type, &extras, &PyTuple_Type, &reductions,
-                        &PyTuple_Type, &outputs))
+  if (!PyArg_ParseTuple(args, "O!y*KiiO!OO!O!O!", &PyTuple_Type, &inputs, &desc, &entry, &left, &right, &PyTuple_Type,
+                        &operands, &tile, &PyTuple_Type, &extras, &PyTuple_Type, &reductions, &PyTuple_Type,
+                        &outputs))
     return nullptr;
+  auto p = std::make_unique<Plan>();
+  const Py_ssize_t desc_len = desc.len;
+  if (desc_len == (Py_ssize_t)sizeof(fuseml_gemm_desc)) std::memcpy(&p->desc, desc.buf, sizeof(fuseml_gemm_desc));
+  PyBuffer_Release(&desc);
   const int n = self->n_inputs;
   if (desc_len != (Py_ssize_t)sizeof(fuseml_gemm_desc) || PyTuple_GET_SIZE(inputs) != n || left < 0 || left >= n ||
       right < 0 || right >= n || PyTuple_GET_SIZE(extras) > FUSEML_MAX_EXTRA_OUT || PyTuple_GET_SIZE(reductions) > 3 ||
@@ -217,13 +220,11 @@ PyObject* launcher_add(PyObject* self_, PyObject* args) {
     return nullptr;
   }
   if (self->plans->size() >= kMaxPlans) Py_RETURN_FALSE;
-  auto p = std::make_unique<Plan>();
   for (int i : *self->used) {
     PyObject* o = PyTuple_GET_ITEM(inputs, i);
     if (!plain(o)) Py_RETURN_FALSE;
     p->signature.push_back(signature_of(THPVariable_Unpack(o)));
   }
-  std::memcpy(&p->desc, desc, sizeof(fuseml_gemm_desc));
   p->entry = reinterpret_cast<Entry>(static_cast<uintptr_t>(entry));
   p->left = left;
   p->right = right;

@@ -345,19 +345,18 @@ class HipKernelLauncher:
         """Hand a plan whose calls need only pointers to the native caller, unless
         its results are cast or viewed after the launch."""
         spec = self.spec
-        if spec.output_shapes or any(dt != torch.float32 for dt in spec.reduce_dtypes):
+        if spec.output_shapes or any(dt is not torch.float32 for dt in spec.reduce_dtypes):
             return
-        desc = _abi.GemmDesc()
-        ctypes.memmove(ctypes.byref(desc), plan.desc_ref, ctypes.sizeof(desc))
-        desc.lda, desc.ldb = plan.lda, plan.ldb
-        entry = self._lib.fuseml_gemm_epilogue_f32 if plan.direct else self._lib.fuseml_gemm_epilogue
-        names = list(spec.reductions)
-        outputs = tuple(("t", 0) if o[0] == "tile" else ("r", names.index(o[1])) if o[0] == "red" else ("e", o[1])
-                        for o in spec.outputs)
-        self._native.add(tuple(inputs), bytes(desc), ctypes.cast(entry, ctypes.c_void_p).value, spec.left, spec.right,
-                         tuple((slot, idx) for slot, (idx, _) in enumerate(plan.operands)),
-                         spec.out_dtype if spec.store_tile else None, tuple(spec.extra_dtypes),
-                         tuple(_abi.RED_SLOT[name] for name in names), outputs)
+        plan.words[_W_LDA], plan.words[_W_LDB] = plan.lda, plan.ldb
+        if plan.single_tile:
+            outputs = (("t", 0),)
+        else:
+            outputs = tuple(("t", 0) if o[0] == "tile" else
+                            ("r", spec.reductions.index(o[1])) if o[0] == "red" else ("e", o[1]) for o in spec.outputs)
+        self._native.add(inputs, plan.desc, _abi.entry_address(plan.direct), spec.left, spec.right,
+                         tuple([(slot, op[0]) for slot, op in enumerate(plan.operands)]),
+                         spec.out_dtype if spec.store_tile else None, spec.extra_dtypes,
+                         tuple([_abi.RED_SLOT[name] for name in spec.reductions]), outputs)
 
     def _launch_fast(self, plan: _Plan, inputs: Sequence[torch.Tensor]) -> Any:
         """A call whose plan needs only pointers: the same checks, allocations
