@@ -418,9 +418,8 @@ constexpr int kRing = 16;                  // weight fragments in flight per wav
 __device__ __forceinline__ int h_chunk(int m, int q) { return m * (kIC * 2) + ((q ^ (m & 15)) << 4); }
 __device__ __forceinline__ int h_byte(int m, int q, int half) { return h_chunk(m, q) + ((half ^ ((m >> 4) & 1)) << 3); }
 
-// PACK: the weight fragments come from d.wpack (fuseml_mlp_pack_weights), one
-// contiguous 1 KB block per fragment, instead of from W1 and W2.
-template <int DW, int GELU, typename T, bool PACK>
+// For weights that are not packed; packed ones run on the eight-wave kernel below.
+template <int DW, int GELU, typename T>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1)))
 void mlp_block_kernel_isplit(const fuseml_mlp_desc d) {
   constexpr int D = 128 * DW;
@@ -453,13 +452,9 @@ void mlp_block_kernel_isplit(const fuseml_mlp_desc d) {
   const uint32_t w1_sc = (uint32_t)kIC * (uint32_t)d.ldw1 * 2u;
   const uint32_t w2_lane = ((uint32_t)(wave * (D / 4) + l32) * (uint32_t)d.ldw2 + (uint32_t)(8 * kh)) * 2u;
   const uint32_t w2_dblk = 32u * (uint32_t)d.ldw2 * 2u;
-  const __amdgpu_buffer_rsrc_t rwp = make_rsrc(d.wpack, PACK ? (int64_t)4 * D * I : 0);
-  const uint32_t wp_lane = (uint32_t)(wave * NF * 1024 + lane * 16);
   auto frag = [&](int c, auto f) -> i32x4_t {
     constexpr int F = decltype(f)::value;
-    if constexpr (PACK) {
-      return __builtin_amdgcn_raw_buffer_load_b128(rwp, wp_lane + (uint32_t)(c * 4 * NF * 1024 + F * 1024), 0, 0);
-    } else if constexpr (F < NF1) {
+    if constexpr (F < NF1) {
       return __builtin_amdgcn_raw_buffer_load_b128(rw1, w1_lane + (uint32_t)c * w1_sc + (uint32_t)(32 * F), 0, 0);
     } else {
       constexpr int s = (F - NF1) / DW, db = (F - NF1) % DW;
@@ -576,28 +571,244 @@ void mlp_block_kernel_isplit(const fuseml_mlp_desc d) {
   }
 }
 
-// fuseml_mlp_pack_weights: block b of the packed buffer is fragment f of wave w
-// of super-chunk c (b = (4 c + w) NF + f, NF = D/8 fragments per wave and
-// super-chunk, in the I-split kernel's consumption order); lane l writes its
-// 16 bytes at b * 1024 + 16 l.  One wave per block.
-__global__ __launch_bounds__(64) void mlp_pack_kernel(const fuseml_mlp_desc d, char* wpack) {
-  const int D = (int)d.D;
-  const int DW = D / 128;
-  const int NF1 = D / 16;
-  const int NF = D / 8;
-  const int b = blockIdx.x;
-  const int c = b / (4 * NF), w = (b / NF) % 4, f = b % NF;
-  const int l32 = threadIdx.x & 31, kh = threadIdx.x >> 5;
-  const uint16_t* src;
-  if (f < NF1) {
-    const int row = kIC * c + 32 * w + l32;
-    src = static_cast<const uint16_t*>(d.w1) + (int64_t)row * d.ldw1 + 16 * f + 8 * kh;
-  } else {
-    const int s = (f - NF1) / DW, db = (f - NF1) % DW;
-    const int row = w * (D / 4) + 32 * db + l32;
-    src = static_cast<const uint16_t*>(d.w2) + (int64_t)row * d.ldw2 + kIC * c + 16 * s + 8 * kh;
+// The block with I split over eight waves, two per SIMD, in two groups that run
+// a super-chunk's phases in a different order, on packed weights (I a multiple of
+// 128; the last super-chunk is packed with zeros past I).  Super-chunk c holds 256 intermediate columns; wave w computes
+// h[rows, 32] of them (GEMM1 over all of D), adds b1, applies GELU and writes
+// them to the LDS h tile, and multiplies the whole h tile by its D/8 rows of W2
+// (GEMM2).  Between two barriers waves 0-3 run GEMM1(c), GELU(c), GEMM2(c - 1)
+// and waves 4-7 GEMM2(c - 1), GEMM1(c), GELU(c): each SIMD holds one wave of
+// each group, so one wave's GELU (VALU) runs beside the other's MFMAs, where the
+// four-wave kernel above runs GEMM1, GELU and GEMM2 one after another on each
+// SIMD (20, 27 and 26% of its time at D = 256, I = 1024, for 26% of MFMA work).
+//   * h is double-buffered: step c writes h(c) and reads h(c - 1), and the buffer
+//     it writes was last read in step c - 1, a barrier earlier.
+//   * A wave's weight fragments lie in its order of consumption, 2 I / 256
+//     segments of D / 16 (fuseml_mlp_pack_weights), and stream through a ring of
+//     registers.
+//   * The MFMA loops of GEMM1 run at raised wave priority: the wave that feeds the
+//     other group's next phase is not held back by GELU instructions.
+// RB: 32-row blocks per workgroup.  Two where every CU gets 64 rows; one below
+// (M <= 32 rows per CU), which halves the MFMA and GELU work of a workgroup for
+// the same weight stream.  What bounds it: at RB = 1 the weight stream (4 D I
+// bytes per workgroup at 55-70 GB/s), at RB = 2 as much the GELU and MFMA issue.
+// Measured (M; D -> I, bf16, us, four waves -> eight): 16384; 256 -> 1024 31.4 ->
+// 27.2, 8192 29.2 -> 18.4, 1000 28.3 -> 16.2; 16384; 512 -> 2048 95.8 -> 77.6,
+// 1000 89.4 -> 47.1.
+constexpr int kIS = 256;                    // intermediate columns per super-chunk
+constexpr int kSkewThreads = 512;
+
+__device__ __forceinline__ int hs_chunk(int m, int q) { return m * (kIS * 2) + ((q ^ (m & 15)) << 4); }
+
+template <int DW, int RB, int GELU, typename T>
+__global__ __launch_bounds__(kSkewThreads) __attribute__((amdgpu_waves_per_eu(2)))
+void mlp_block_kernel_skew(const fuseml_mlp_desc d) {
+  constexpr int D = 128 * DW;
+  constexpr int PITCH = 2 * D;
+  constexpr int BM = 32 * RB;
+  // 16 fragments in flight per wave; 8 where the accumulators leave no registers.
+  constexpr int RING = DW * RB > 4 ? 8 : 16;
+  constexpr int NS = D / 16;       // weight fragments per segment: GEMM1's, and GEMM2's
+  constexpr int DB = D / 256;      // 32-column blocks of y per wave
+  constexpr int kH = BM * kIS * 2; // one h tile
+  static_assert(NS % RING == 0 && (kIS / 16) * DB == NS, "segments are whole ring turns");
+  __shared__ __attribute__((aligned(1024))) char smem[BM * PITCH + 2 * kH];
+  char* xs = smem;
+  char* hs = smem + BM * PITCH;
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int l32 = lane & 31;
+  const int kh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool late = wave >= 4;     // this wave's group runs GEMM2 first
+  const int M = (int)d.M, I = (int)d.I;
+  const int nblocks = (M + BM - 1) / BM;
+  const int nsc = (I + kIS - 1) / kIS;
+
+  const __amdgpu_buffer_rsrc_t rb1 = make_rsrc(d.b1, (int64_t)I * 2);
+  // This wave's stream: 2 nsc segments of NS KB.
+  const int stream = 2 * nsc * NS * 1024;
+  const __amdgpu_buffer_rsrc_t rwp = make_rsrc(static_cast<const char*>(d.wpack) + (int64_t)wave * stream, stream);
+  const uint32_t wl = (uint32_t)(lane * 16);
+  i32x4_t ring[RING];
+
+  for (int blk = blockIdx.x; blk < nblocks; blk += gridDim.x) {
+    const int m0 = blk * BM;
+    if (blk != (int)blockIdx.x) barrier();  // the previous block no longer reads x or h
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    {
+      const __amdgpu_buffer_rsrc_t rx = make_rsrc(static_cast<const char*>(d.x) + (int64_t)m0 * d.ldx * 2,
+                                                  ((int64_t)(M - 1 - m0) * d.ldx + D) * 2);
+      constexpr int kDmas = BM * PITCH / 1024;
+      for (int i = wave; i < kDmas; i += 8) {
+        const int byte = i * 1024 + ln * 16;
+        const int m = byte / PITCH;
+        const int q = ((byte % PITCH) >> 4) ^ (m & 15);
+        const uint32_t off = m0 + m < M ? ((uint32_t)m * (uint32_t)d.ldx + (uint32_t)(8 * q)) * 2u : kOOB;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (__attribute__((address_space(3))) void*)(xs + i * 1024), 16, off,
+                                                 0, 0, 0);
+      }
+    }
+    int pos = 0;  // byte offset of the current segment in the stream
+    static_for<0, RING>([&](auto f) { ring[f] = __builtin_amdgcn_raw_buffer_load_b128(rwp, wl, f * 1024, 0); });
+    f32x16_t acc[RB][DB];
+    static_for<0, RB>([&](auto mb) {
+      static_for<0, DB>([&](auto db) { static_for<0, 16>([&](auto r) { acc[mb][db][(int)r] = 0.0f; }); });
+    });
+    wait_vmcnt0();
+    barrier();  // x tile landed
+
+    // Fragment f of the current segment, its slot refilled with the fragment
+    // RING further on (past the end of the stream: the first one, not used).
+    auto take = [&](auto f) {
+      const i32x4_t w = ring[f % RING];
+      int next = pos + (f + RING) * 1024;
+      if constexpr (f + RING >= NS) next = next < stream ? next : 0;
+      ring[f % RING] = __builtin_amdgcn_raw_buffer_load_b128(rwp, wl, next, 0);
+      return w;
+    };
+    auto gemm1 = [&](int c) {
+      i32x2_t bq[4];
+      static_for<0, 4>([&](auto g) {
+        bq[g] = __builtin_amdgcn_raw_buffer_load_b64(rb1, (uint32_t)(c * kIS + 32 * wave + 8 * g + 4 * kh) * 2u, 0, 0);
+      });
+      f32x16_t h1[RB];
+      static_for<0, RB>([&](auto mb) { static_for<0, 16>([&](auto r) { h1[mb][(int)r] = 0.0f; }); });
+      __builtin_amdgcn_s_setprio(1);
+      static_for<0, NS>([&](auto s) {
+        const i32x4_t w = take(s);
+        static_for<0, RB>([&](auto mb) {
+          const int m = 32 * mb + l32;
+          const i32x4_t xf = *reinterpret_cast<const i32x4_t*>(xs + x_chunk(m, 2 * s + kh, PITCH));
+          h1[mb] = mfma32<T>(w, xf, h1[mb]);
+        });
+      });
+      __builtin_amdgcn_s_setprio(0);
+      pos += NS * 1024;
+      // h1[mb][r] = h[32 mb + l32][32 wave + 8 (r>>2) + 4 kh + (r&3)]
+      char* hb = hs + (c & 1) * kH;
+      float v[16 * RB];
+      static_for<0, RB>([&](auto mb) {
+        static_for<0, 4>([&](auto g) {
+          static_for<0, 4>([&](auto e) {
+            const uint32_t bw = (uint32_t)(e < 2 ? bq[g].x : bq[g].y) >> (16 * (e & 1));
+            const float t = h1[mb][4 * g + e] + to_f32<T>(bw & 0xffffu);
+            v[16 * mb + 4 * g + e] = GELU == FUSEML_OP_GELU_TANH ? gelu_tanh(t) : gelu_erf(t);
+          });
+        });
+      });
+      post_ops<16 * RB>(d, v);
+      static_for<0, RB>([&](auto mb) {
+        const int m = 32 * mb + l32;
+        static_for<0, 4>([&](auto g) {
+          constexpr int o = 16 * mb + 4 * g;
+          const i32x2_t hv = {(int)pack2<T>(v[o], v[o + 1]), (int)pack2<T>(v[o + 2], v[o + 3])};
+          *reinterpret_cast<i32x2_t*>(hb + hs_chunk(m, 4 * wave + g) + ((kh ^ ((m >> 4) & 1)) << 3)) = hv;
+        });
+      });
+    };
+    auto gemm2 = [&](int c) {
+      const char* hb = hs + (c & 1) * kH;
+      static_for<0, kIS / 16>([&](auto s) {
+        i32x4_t hf[RB];
+        static_for<0, RB>([&](auto mb) {
+          const int m = 32 * mb + l32;
+          i32x4_t x = *reinterpret_cast<const i32x4_t*>(hb + hs_chunk(m, 2 * s + kh));
+          if ((m >> 4) & 1) x = i32x4_t{x.z, x.w, x.x, x.y};
+          hf[mb] = x;
+        });
+        static_for<0, DB>([&](auto db) {
+          const i32x4_t w = take(std::integral_constant<int, DB * decltype(s)::value + decltype(db)::value>{});
+          static_for<0, RB>([&](auto mb) { acc[mb][db] = mfma32<T>(w, hf[mb], acc[mb][db]); });
+        });
+      });
+      pos += NS * 1024;
+    };
+
+    gemm1(0);
+    barrier();
+    for (int c = 1; c < nsc; ++c) {
+      if (late) gemm2(c - 1);
+      gemm1(c);
+      if (!late) gemm2(c - 1);
+      barrier();  // h(c) complete, h(c - 1) read
+    }
+    gemm2(nsc - 1);
+
+    // y = acc + b2 + r; acc[mb][db][r] is y[m0 + 32 mb + l32][wave D/8 + 32 db +
+    // 8 (r>>2) + 4 kh + (r&3)].
+    const __amdgpu_buffer_rsrc_t rb2 = make_rsrc(d.b2, d.b2 ? (int64_t)D * 2 : 0);
+    const __amdgpu_buffer_rsrc_t rr = make_rsrc(
+        d.r ? static_cast<const char*>(d.r) + (int64_t)m0 * d.ldr * 2 : nullptr,
+        d.r ? ((int64_t)(M - 1 - m0) * d.ldr + D) * 2 : 0);
+    const __amdgpu_buffer_rsrc_t ry =
+        make_rsrc(static_cast<char*>(d.y) + (int64_t)m0 * d.ldy * 2, ((int64_t)(M - 1 - m0) * d.ldy + D) * 2);
+    const int el32 = ln & 31, ekh = ln >> 5;
+    i32x2_t bv[DB][4], rv[RB][DB][4];
+    static_for<0, DB>([&](auto db) {
+      static_for<0, 4>([&](auto g) {
+        const int col = wave * (D / 8) + 32 * db + 8 * g + 4 * ekh;
+        bv[db][g] = __builtin_amdgcn_raw_buffer_load_b64(rb2, (uint32_t)col * 2u, 0, 0);
+        static_for<0, RB>([&](auto mb) {
+          const int ml = 32 * mb + el32;
+          rv[mb][db][g] = __builtin_amdgcn_raw_buffer_load_b64(
+              rr, m0 + ml < M ? ((uint32_t)ml * (uint32_t)d.ldr + (uint32_t)col) * 2u : kOOB, 0, 0);
+        });
+      });
+    });
+    static_for<0, RB>([&](auto mb) {
+      const int ml = 32 * mb + el32;
+      static_for<0, DB>([&](auto db) {
+        static_for<0, 4>([&](auto g) {
+          const int col = wave * (D / 8) + 32 * db + 8 * g + 4 * ekh;
+          float y[4];
+          static_for<0, 4>([&](auto e) {
+            const uint32_t bw = (uint32_t)(e < 2 ? bv[db][g].x : bv[db][g].y) >> (16 * (e & 1));
+            const uint32_t rw = (uint32_t)(e < 2 ? rv[mb][db][g].x : rv[mb][db][g].y) >> (16 * (e & 1));
+            y[e] = acc[mb][db][4 * g + e] + to_f32<T>(bw & 0xffffu) + to_f32<T>(rw & 0xffffu);
+          });
+          const i32x2_t out = {(int)pack2<T>(y[0], y[1]), (int)pack2<T>(y[2], y[3])};
+          __builtin_amdgcn_raw_buffer_store_b64(
+              out, ry, m0 + ml < M ? ((uint32_t)ml * (uint32_t)d.ldy + (uint32_t)col) * 2u : kOOB, 0, 0);
+        });
+      });
+    });
   }
-  *reinterpret_cast<i32x4_t*>(wpack + (int64_t)b * 1024 + threadIdx.x * 16) = *reinterpret_cast<const i32x4_t*>(src);
+}
+
+// fuseml_mlp_pack_weights, the order of the kernel above: block b is fragment f of segment q of
+// wave w's stream (b = (2 nsc w + q) NS + f).  Segment 0 is W1 of super-chunk 0;
+// then, per super-chunk c >= 1, W1(c) and W2(c - 1) for waves 0-3, W2(c - 1) and
+// W1(c) for waves 4-7; the last is W2 of the last super-chunk.
+__global__ __launch_bounds__(64) void mlp_pack_kernel(const fuseml_mlp_desc d, char* wpack) {
+  const int D = (int)d.D, NS = D / 16, DB = D / 256;
+  const int I = (int)d.I;
+  const int nsc = (I + kIS - 1) / kIS;
+  const int b = blockIdx.x;
+  const int f = b % NS, q = (b / NS) % (2 * nsc), w = b / (2 * nsc * NS);
+  const int l32 = threadIdx.x & 31, kh = threadIdx.x >> 5;
+  const bool first = q == 0, last = q == 2 * nsc - 1;
+  const bool odd = (q & 1) != 0;                         // segments 2 c - 1, 2 c: step c
+  const bool is_w1 = first || (!last && (odd == (w < 4)));
+  const int step = (q + 1) / 2;                          // q = 2 c - 1 or 2 c -> c
+  // Rows of W1 and columns of W2 past I are zeros (I is a multiple of 128, so a
+  // fragment lies wholly on one side).
+  const uint16_t* src = nullptr;
+  if (is_w1) {
+    const int c = first ? 0 : step;
+    if (kIS * c + 32 * w < I)
+      src = static_cast<const uint16_t*>(d.w1) + (int64_t)(kIS * c + 32 * w + l32) * d.ldw1 + 16 * f + 8 * kh;
+  } else {
+    const int c = last ? nsc - 1 : step - 1;
+    const int s = f / DB, db = f % DB;
+    if (kIS * c + 16 * s < I)
+      src = static_cast<const uint16_t*>(d.w2) + (int64_t)(w * (D / 8) + 32 * db + l32) * d.ldw2 + kIS * c + 16 * s + 8 * kh;
+  }
+  i32x4_t x = {0, 0, 0, 0};
+  if (src != nullptr) x = *reinterpret_cast<const i32x4_t*>(src);
+  *reinterpret_cast<i32x4_t*>(wpack + (int64_t)b * 1024 + threadIdx.x * 16) = x;
 }
 
 void set_error(const char* msg) { fuseml_detail::set_error_text(msg); }
@@ -625,6 +836,9 @@ int device_cus(int dev) {
   if (dev >= 0 && dev < kMaxDevices) g_cus[dev].store(cus, std::memory_order_relaxed);
   return cus;
 }
+
+// Bytes of the packed weights: W1 and W2 with I rounded up to whole super-chunks.
+int64_t packed_bytes(const fuseml_mlp_desc& d) { return 4 * d.D * ((d.I + kIS - 1) / kIS * kIS); }
 
 int validate(const fuseml_mlp_desc* dp) {
   if (dp == nullptr) {
@@ -670,7 +884,7 @@ int validate(const fuseml_mlp_desc* dp) {
     set_error("mlp_block: strides or alignment not supported");
     return FUSEML_EUNSUPPORTED;
   }
-  if (d.wpack != nullptr && (((uintptr_t)d.wpack & 15) || (int64_t)4 * d.D * d.I >= ((int64_t)1 << 31))) {
+  if (d.wpack != nullptr && (((uintptr_t)d.wpack & 15) || packed_bytes(d) >= ((int64_t)1 << 31))) {
     set_error("mlp_block: packed weights misaligned or 2 GiB or more");
     return FUSEML_EUNSUPPORTED;
   }
@@ -695,22 +909,34 @@ bool use_isplit(const fuseml_mlp_desc& d) {
   return d.I % kIC == 0 && d.D <= 512 && !force_dsplit;
 }
 
+template <int DW, int RB, typename T>
+hipError_t launch_skew(const fuseml_mlp_desc& d, int cus, hipStream_t s) {
+  const int64_t blocks = (d.M + 32 * RB - 1) / (32 * RB);
+  const dim3 grid((unsigned)(blocks < cus ? blocks : cus)), block(kSkewThreads);
+  if (d.gelu == FUSEML_OP_GELU_TANH)
+    hipLaunchKernelGGL((mlp_block_kernel_skew<DW, RB, FUSEML_OP_GELU_TANH, T>), grid, block, 0, s, d);
+  else
+    hipLaunchKernelGGL((mlp_block_kernel_skew<DW, RB, FUSEML_OP_GELU_ERF, T>), grid, block, 0, s, d);
+  return hipGetLastError();
+}
+
 template <int DW, typename T>
-hipError_t launch_dw(const fuseml_mlp_desc& d, int grid, hipStream_t s) {
+hipError_t launch_dw(const fuseml_mlp_desc& d, int cus, hipStream_t s) {
   const bool tanh_gelu = d.gelu == FUSEML_OP_GELU_TANH;
+  if constexpr (DW <= 4) {
+    if (d.wpack != nullptr && use_isplit(d))
+      return d.M <= 32 * (int64_t)cus ? launch_skew<DW, 1, T>(d, cus, s) : launch_skew<DW, 2, T>(d, cus, s);
+  }
+  const int64_t nblocks = (d.M + kBM - 1) / kBM;
+  const int grid = (int)(nblocks < cus ? nblocks : cus);
   // D = 1024 stays on the D-split kernel: the I-split one's 64 x 1024
   // accumulators and weight ring do not fit the register file.
   if constexpr (DW <= 4) {
     if (use_isplit(d)) {
-      const bool pack = d.wpack != nullptr;
-      if (tanh_gelu && pack)
-        hipLaunchKernelGGL((mlp_block_kernel_isplit<DW, FUSEML_OP_GELU_TANH, T, true>), dim3(grid), dim3(kThreads), 0, s, d);
-      else if (tanh_gelu)
-        hipLaunchKernelGGL((mlp_block_kernel_isplit<DW, FUSEML_OP_GELU_TANH, T, false>), dim3(grid), dim3(kThreads), 0, s, d);
-      else if (pack)
-        hipLaunchKernelGGL((mlp_block_kernel_isplit<DW, FUSEML_OP_GELU_ERF, T, true>), dim3(grid), dim3(kThreads), 0, s, d);
+      if (tanh_gelu)
+        hipLaunchKernelGGL((mlp_block_kernel_isplit<DW, FUSEML_OP_GELU_TANH, T>), dim3(grid), dim3(kThreads), 0, s, d);
       else
-        hipLaunchKernelGGL((mlp_block_kernel_isplit<DW, FUSEML_OP_GELU_ERF, T, false>), dim3(grid), dim3(kThreads), 0, s, d);
+        hipLaunchKernelGGL((mlp_block_kernel_isplit<DW, FUSEML_OP_GELU_ERF, T>), dim3(grid), dim3(kThreads), 0, s, d);
       return hipGetLastError();
     }
   }
@@ -723,11 +949,11 @@ hipError_t launch_dw(const fuseml_mlp_desc& d, int grid, hipStream_t s) {
 }
 
 template <typename T>
-hipError_t launch_t(const fuseml_mlp_desc& d, int grid, hipStream_t s) {
+hipError_t launch_t(const fuseml_mlp_desc& d, int cus, hipStream_t s) {
   switch (d.D) {
-    case 256: return launch_dw<2, T>(d, grid, s);
-    case 512: return launch_dw<4, T>(d, grid, s);
-    default: return launch_dw<8, T>(d, grid, s);
+    case 256: return launch_dw<2, T>(d, cus, s);
+    case 512: return launch_dw<4, T>(d, cus, s);
+    default: return launch_dw<8, T>(d, cus, s);
   }
 }
 
@@ -744,7 +970,7 @@ int64_t fuseml_mlp_pack_bytes(const fuseml_mlp_desc* desc) {
   set_error("");
   if (validate(desc) != FUSEML_OK) return 0;
   if (!(desc->D == 256 || desc->D == 512) || desc->I % kIC != 0) return 0;
-  return (int64_t)4 * desc->D * desc->I;
+  return packed_bytes(*desc);
 }
 
 int fuseml_mlp_pack_weights(const fuseml_mlp_desc* desc, void* wpack, void* stream) {
@@ -766,9 +992,9 @@ int fuseml_mlp_pack_weights(const fuseml_mlp_desc* desc, void* wpack, void* stre
   }
   const int cus = device_cus(dev);
   if (cus <= 0) return cus < 0 ? cus : FUSEML_EHIP;
-  const int64_t blocks = (desc->I / kIC) * 4 * (desc->D / 8);
-  hipLaunchKernelGGL(mlp_pack_kernel, dim3((unsigned)blocks), dim3(64), 0, reinterpret_cast<hipStream_t>(stream), *desc,
-                     static_cast<char*>(wpack));
+  const int64_t blocks = packed_bytes(*desc) / 1024;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  hipLaunchKernelGGL(mlp_pack_kernel, dim3((unsigned)blocks), dim3(64), 0, s, *desc, static_cast<char*>(wpack));
   if (hipGetLastError() != hipSuccess) {
     set_error("mlp_pack_weights launch failed");
     return FUSEML_EHIP;
@@ -787,10 +1013,8 @@ int fuseml_mlp_block(const fuseml_mlp_desc* desc, void* stream) {
   }
   const int cus = device_cus(dev);
   if (cus <= 0) return cus < 0 ? cus : FUSEML_EHIP;
-  const int64_t nblocks = (desc->M + kBM - 1) / kBM;
-  const int grid = (int)(nblocks < cus ? nblocks : cus);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const hipError_t e = desc->dtype == FUSEML_BF16 ? launch_t<__bf16>(*desc, grid, s) : launch_t<_Float16>(*desc, grid, s);
+  const hipError_t e = desc->dtype == FUSEML_BF16 ? launch_t<__bf16>(*desc, cus, s) : launch_t<_Float16>(*desc, cus, s);
   if (e != hipSuccess) {
     set_error("mlp_block launch failed");
     return FUSEML_EHIP;
