@@ -278,14 +278,20 @@ def entry_address(f32: bool) -> int:
     return _entries[f32]
 
 
+_fast_launcher = None
+
+
 def load_fastcall():
-    """The launchers' native-call extension; ImportError if it is not built."""
-    try:
-        from . import _fastcall
-    except ImportError as exc:
-        raise ImportError(f"fuseml_amd/_fastcall.so cannot be loaded ({exc}) — run `python -m fuseml_amd.build` "
-                          "(or __graft_entry__.build()) first") from exc
-    return _fastcall
+    """The native caller's type (csrc/fastcall.cpp); ImportError if it is not built."""
+    global _fast_launcher
+    if _fast_launcher is None:
+        try:
+            from . import _fastcall
+        except ImportError as exc:
+            raise ImportError(f"fuseml_amd/_fastcall.so cannot be loaded ({exc}) — run `python -m fuseml_amd.build` "
+                              "(or __graft_entry__.build()) first") from exc
+        _fast_launcher = _fastcall.Launcher
+    return _fast_launcher
 
 
 VARIANTS = ("large", "deep", "deep3", "small", "narrow64", "narrow32", "large128", "small64")

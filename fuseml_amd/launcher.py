@@ -105,6 +105,12 @@ assert all(o % _WORD == 0 for o in (_abi.GemmDesc.a.offset, _abi.GemmDesc.operan
                                      _abi.GemmDesc.reduce_out.offset, ctypes.sizeof(_abi.GemmDesc)))
 
 
+# A signature's calls run in native code after this many: handing a plan over costs
+# some microseconds (tens in a process whose caches hold other work), which a
+# signature that is seen once or twice would not get back.
+_NATIVE_AFTER = 3
+
+
 class _Plan:
     """What a launch needs that depends only on the input signature (shapes,
     strides, dtypes): the descriptor with every non-pointer field filled, M/N/K,
@@ -124,7 +130,7 @@ class _Plan:
 
     __slots__ = ("desc", "M", "N", "K", "neg", "operands", "nbytes", "k_split", "fast", "words", "desc_ref",
                  "a_ok", "b_ok", "lda", "ldb", "op_words", "red_words", "extra_words", "single_tile", "direct",
-                 "split_plan", "native")
+                 "split_plan", "calls")
 
     def __init__(self) -> None:
         self.desc = _abi.GemmDesc()
@@ -146,7 +152,7 @@ class _Plan:
         self.single_tile = False
         self.direct = False
         self.split_plan: Optional["_Plan"] = None
-        self.native: Optional[bool] = None  # handed to the native caller; None: its signature was seen once
+        self.calls = 0  # fast calls made in Python
 
 
 class HipKernelLauncher:
@@ -179,9 +185,9 @@ class HipKernelLauncher:
         self.timing_pool: List[Tuple[Any, Any]] = []
         # Input slots the launch reads: the GEMM operands and the epilogue operands.
         self._used = sorted({spec.left, spec.right} | {op.operand for op in spec.ops if op.kind in ("add", "mul")})
-        # Later calls of a signature whose plan needs only pointers run in native
+        # Repeated calls of a signature whose plan needs only pointers run in native
         # code (csrc/fastcall.cpp); it declines every other call.
-        self._native = _abi.load_fastcall().Launcher(n_inputs, tuple(self._used), self._fallback_guard is not None)
+        self._native = _abi.load_fastcall()(n_inputs, tuple(self._used), self._fallback_guard is not None)
         self._native_call = self._native.call
 
     # ------------------------------------------------------------------
@@ -326,11 +332,6 @@ class HipKernelLauncher:
         if plan is None:
             plan = self._make_plan(inputs)
             self._plans[key] = plan
-        elif plan.native is None:
-            # The signature came back: its next calls run in native code.
-            plan.native = plan.fast and plan.a_ok and plan.b_ok and isinstance(self._lib, ctypes.CDLL)
-            if plan.native:
-                self._add_native(plan, inputs)
         if plan.direct and (inputs[self.spec.left].data_ptr() | inputs[self.spec.right].data_ptr()) % 16:
             if plan.split_plan is None:
                 plan.split_plan = self._make_plan(inputs, allow_direct=False)
@@ -338,7 +339,12 @@ class HipKernelLauncher:
         # (tests may bind a recorder as the library: the general path, which
         # assumes no device, serves those)
         if plan.fast and self.timing_events is None and isinstance(self._lib, ctypes.CDLL):
-            return self._launch_fast(plan, inputs)
+            out = self._launch_fast(plan, inputs)
+            plan.calls += 1
+            if plan.calls == _NATIVE_AFTER and plan.a_ok and plan.b_ok:
+                # While the GPU works on this call.
+                self._add_native(plan, inputs)
+            return out
         return self._launch_general(plan, inputs)
 
     def _add_native(self, plan: _Plan, inputs: Sequence[torch.Tensor]) -> None:

@@ -13,7 +13,7 @@ import torch
 from fuseml_amd import _abi
 from fuseml_amd.epilogue import EpilogueSpec, EpiOp
 from fuseml_amd.fallback import FORCE_FAIL_ENV
-from fuseml_amd.launcher import HipKernelLauncher
+from fuseml_amd.launcher import _NATIVE_AFTER, HipKernelLauncher
 
 BF = torch.bfloat16
 SPEC = EpilogueSpec(1, 2, (EpiOp("add", 0), EpiOp("gelu_erf")), BF)
@@ -26,7 +26,7 @@ def _args(M=32, N=264, K=128, device="cpu", dtype=BF):
 
 
 def test_host_tensors_and_unknown_calls_are_declined():
-    fast = _abi.load_fastcall().Launcher(3, (0, 1, 2), False)
+    fast = _abi.load_fastcall()(3, (0, 1, 2), False)
     args = _args()
     assert fast.call(args) is None and fast.call(args[:2]) is None and fast.call([*args]) is None
     desc = bytes(_abi.GemmDesc())
@@ -42,7 +42,7 @@ def test_host_tensors_and_unknown_calls_are_declined():
 def test_malformed_plans_are_refused(bad):
     """No plan reaches the list whose call could write outside its descriptor
     (with tensors a plan is not taken for, so a wrong acceptance shows as False)."""
-    fast = _abi.load_fastcall().Launcher(3, (0, 1, 2), False)
+    fast = _abi.load_fastcall()(3, (0, 1, 2), False)
     a = dict(desc=bytes(_abi.GemmDesc()), left=1, right=2, operands=((0, 0),), extras=(), reductions=(),
              outputs=(("t", 0),)) | bad
     checked_late = {"operands", "outputs"} & set(bad) or bad.get("reductions") == (3,)
@@ -70,8 +70,9 @@ def test_native_call_is_the_python_call(dtype):
     L = HipKernelLauncher(spec, 3)
     for M, N in ((32, 264), (300, 520), (32, 264), (1, 8)):
         args = _args(M, N, device="cuda", dtype=dtype)
-        first = L(*args)             # a new signature: Python makes its plan,
-        L(*args)                     # and hands it over when it comes back
+        first = L(*args)
+        for _ in range(_NATIVE_AFTER - 1):
+            L(*args)                 # then the signature's plan is handed over
         before = L._native.count
         got = L(*args)
         assert L._native.count == before + 1
@@ -81,7 +82,7 @@ def test_native_call_is_the_python_call(dtype):
             torch.testing.assert_close(g, w, rtol=1e-6, atol=1e-6)  # fp32 sums by atomics
             torch.testing.assert_close(f, w, rtol=1e-6, atol=1e-6)
         assert got[1].data_ptr() != first[1].data_ptr()
-    assert L.launch_count == 4 * 4
+    assert L.launch_count == 4 * (_NATIVE_AFTER + 2)
 
 
 @gpu
@@ -91,8 +92,8 @@ def test_declined_forms_give_the_same_result():
     L = HipKernelLauncher(SPEC, 3, eager_fn=lambda b, x, w: torch.nn.functional.gelu(torch.addmm(b, x, w)))
     b, x, wt = _args(device="cuda")
     want = L(b, x, wt)
-    L(b, x, wt)
-    L(b, x, wt)
+    for _ in range(_NATIVE_AFTER):
+        L(b, x, wt)
     n = L._native.count
     assert n == 1
     off = torch.empty(x.shape[0], x.shape[1] + 8, dtype=BF, device="cuda")[:, 3:-5].copy_(x)
@@ -134,9 +135,9 @@ def test_more_signatures_than_native_plans():
     b, x, wt = _args(M=200, device="cuda")
     full = L(b, x, wt)
     for m in range(1, 100):
-        for _ in range(3):
+        for _ in range(_NATIVE_AFTER + 1):
             torch.testing.assert_close(L(b, x[:m], wt).float(), full[:m].float(), rtol=2 ** -7, atol=2 ** -7)
-    assert L.launch_count == 1 + 3 * 99 and L._native.count == 64
+    assert L.launch_count == 1 + (_NATIVE_AFTER + 1) * 99 and L._native.count == 64
 
 
 @gpu
@@ -171,7 +172,7 @@ def test_threads_and_streams_share_a_launcher():
 def test_native_call_in_a_graph_replays():
     L = HipKernelLauncher(SPEC, 3)
     b, x, wt = _args(device="cuda")
-    for _ in range(3):
+    for _ in range(_NATIVE_AFTER + 1):
         L(b, x, wt)
     assert L._native.count == 1
     torch.cuda.synchronize()
