@@ -698,7 +698,10 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
     constexpr int RPS = STAGE / SP;   // staging rows per pipeline slot
     static_assert(!kOpDma || (STAGE % SP == 0 && RPS % 32 == 0 && RPS == RPD * NW * LPS),
                   "operand DMAs line up with the stage DMAs");
-    const bool op_dma = kOpDma && staged >= 0 && (d.operands[staged].reserved & kFlagAligned) != 0;
+    // (flags read once, here: a scalar load behind the K loop waits for memory)
+    const bool staged_aligned = staged >= 0 && (d.operands[staged].reserved & kFlagAligned) != 0;
+    const bool op_dma = kOpDma && staged_aligned;
+    const int out_flags = d.out.reserved;
     const void* op_ptr = d.a;
     int64_t op_bytes = 0;  // bytes of the operand from its row m0 on
     uint32_t op_o[kOpDma ? LPS : 1];  // chunk c's byte offset in its slot (kOOB: column past N)
@@ -1273,7 +1276,7 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
       constexpr int NP = BM / RPP;
       constexpr int PB = NP < 8 ? NP : 8;
       static_assert(NP % PB == 0, "pass batches");
-      if (d.operands[staged].reserved & kFlagAligned) {
+      if (staged_aligned) {
         static_for<0, NP / PB>([&](auto b) {
           i32x4_t x[PB];
           static_for<0, PB>([&](auto q) {
@@ -1326,7 +1329,7 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
     // vector's values (which depend only on the column) are read from LDS once
     // per column block.  Carrying one column block (not all of them) through the
     // runtime op loop keeps the loop's live values within the register file.
-    const bool use_stage_out = d.out.ptr != nullptr && (d.out.reserved & kFlagStage);
+    const bool use_stage_out = d.out.ptr != nullptr && (out_flags & kFlagStage);
     // Activations run a step at a time across EW values (independent VALU
     // chains).  16 instead of 8 for the one-wave schedule measured no faster.
     constexpr int EW = 8;
@@ -1774,7 +1777,7 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
       // 16 passes unrolled: their LDS reads are in flight together (measured 2%
       // faster than 4 at 16384x4096x1024 with no ops; the kernel's code is small
       // enough since the column blocks share one copy of the op code).
-      if (d.out.reserved & kFlagAligned) {
+      if (out_flags & kFlagAligned) {
 #pragma unroll 16
         for (int p = 0; p < BM / RPP; ++p) {
           const int rl = p * RPP + crow;
