@@ -620,6 +620,7 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
     const int wm = wave / WN;
     const int wn = wave % WN;
     const int M = (int)d.M, N = (int)d.N, K = (int)d.K;
+    int out_flags = d.out.reserved;
     const int strip = kGroupM * tiles_n;
     const int first_m = (lid / strip) * kGroupM;
     const int strip_h = min(tiles_m - first_m, kGroupM);
@@ -671,11 +672,14 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
 
     // The epilogue stages the first LDS-eligible 2-D operand of the chain in an
     // LDS tile [BM][BN] of 16-bit elements that reuses the pipeline's slots.
-    int staged = -1;
+    int staged = -1, staged_flags = 0;
     for (int o = 0; o < d.n_ops; ++o) {
       const int k = d.ops[o].kind;
-      if ((k == FUSEML_OP_ADD || k == FUSEML_OP_MUL) && (d.operands[d.ops[o].operand].reserved & kFlagStage)) {
+      if (k != FUSEML_OP_ADD && k != FUSEML_OP_MUL) continue;
+      const int fl = d.operands[d.ops[o].operand].reserved;
+      if (fl & kFlagStage) {
         staged = d.ops[o].operand;
+        staged_flags = fl;
         break;
       }
     }
@@ -698,10 +702,8 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
     constexpr int RPS = STAGE / SP;   // staging rows per pipeline slot
     static_assert(!kOpDma || (STAGE % SP == 0 && RPS % 32 == 0 && RPS == RPD * NW * LPS),
                   "operand DMAs line up with the stage DMAs");
-    // (flags read once, here: a scalar load behind the K loop waits for memory)
-    const bool staged_aligned = staged >= 0 && (d.operands[staged].reserved & kFlagAligned) != 0;
+    const bool staged_aligned = (staged_flags & kFlagAligned) != 0;
     const bool op_dma = kOpDma && staged_aligned;
-    const int out_flags = d.out.reserved;
     const void* op_ptr = d.a;
     int64_t op_bytes = 0;  // bytes of the operand from its row m0 on
     uint32_t op_o[kOpDma ? LPS : 1];  // chunk c's byte offset in its slot (kOOB: column past N)
@@ -836,6 +838,12 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
     // Fragment row byte offsets inside a stage: rows of W feed MFMA "A", rows of x MFMA "B".
     const int fa_row = A_BYTES + (wn * TN + l32) * RB;
     const int fb_row = (wm * TM + l32) * RB;
+
+    // The output's flags have arrived before the K loop (the empty asm uses them): a
+    // scalar load behind the loop waits for memory, and one still pending at its
+    // entry turns the loop's counted LDS waits into full ones, since scalar loads
+    // return out of order (64x128 tiles at K = 4096: 1.4%).
+    asm volatile("" : "+s"(out_flags));
 
     // MFMAs of one stage.  Fragments of k-step ks+1 are read from LDS while the
     // MFMAs of k-step ks run.
