@@ -23,6 +23,7 @@ kernel_launcher.py:496-509, 816-821, extended to sum and amax).
 from __future__ import annotations
 
 import ctypes
+import threading
 from typing import Any, Callable, Dict, List, Optional, Sequence, Tuple
 
 import torch
@@ -109,6 +110,7 @@ assert all(o % _WORD == 0 for o in (_abi.GemmDesc.a.offset, _abi.GemmDesc.operan
 # some microseconds (tens in a process whose caches hold other work), which a
 # signature that is seen once or twice would not get back.
 _NATIVE_AFTER = 3
+_native_lock = threading.Lock()
 
 
 class _Plan:
@@ -187,13 +189,14 @@ class HipKernelLauncher:
         self._used = sorted({spec.left, spec.right} | {op.operand for op in spec.ops if op.kind in ("add", "mul")})
         # Repeated calls of a signature whose plan needs only pointers run in native
         # code (csrc/fastcall.cpp); it declines every other call.
-        self._native = _abi.load_fastcall()(n_inputs, tuple(self._used), self._fallback_guard is not None)
-        self._native_call = self._native.call
+        self._native_type = _abi.load_fastcall()
+        self._native: Optional[Any] = None  # made with the first plan handed over
+        self._native_call: Optional[Callable[..., Any]] = None
 
     # ------------------------------------------------------------------
     @property
     def launch_count(self) -> int:
-        return self._python_launches + self._native.count
+        return self._python_launches + (self._native.count if self._native is not None else 0)
 
     @property
     def fallback_count(self) -> int:
@@ -353,6 +356,10 @@ class HipKernelLauncher:
         spec = self.spec
         if spec.output_shapes or any(dt is not torch.float32 for dt in spec.reduce_dtypes):
             return
+        with _native_lock:  # one per launcher: it holds the launch count
+            if self._native is None:
+                self._native = self._native_type(self._n_inputs, tuple(self._used), self._fallback_guard is not None)
+                self._native_call = self._native.call
         plan.words[_W_LDA], plan.words[_W_LDB] = plan.lda, plan.ldb
         if plan.single_tile:
             outputs = (("t", 0),)
@@ -459,7 +466,7 @@ class HipKernelLauncher:
             return self._assemble(tile, extras, reds)
 
         d = plan.desc
-        stream = torch.cuda.current_stream(dev).cuda_stream if dev.type == "cuda" else 0
+        stream = torch._C._cuda_getCurrentRawStream(dev.index) if dev.type == "cuda" else 0
         if plan.k_split:
             a, b = self._split_operands(plan, a, b, stream)
             d.a, d.lda = a.data_ptr(), a.stride(0)
@@ -539,7 +546,7 @@ class HipKernelLauncher:
 
     # ------------------------------------------------------------------
     def __call__(self, *inputs: torch.Tensor) -> Any:
-        if self.timing_events is None:
+        if self._native_call is not None and self.timing_events is None:
             try:
                 out = self._native_call(inputs)
                 if type(out) is int:
