@@ -188,6 +188,37 @@ def _gemm_dims(group: Any) -> Tuple[Optional[int], Any, Optional[int], Optional[
 # eager's time at K = 2048-4096, 1.07 at K = 8192).
 WEIGHT_STREAM_K_PER_PASS = 4096
 
+# The library's K-split tiles (kKsplit in csrc/gemm_epilogue_shared.h): 16-row and
+# 16-column blocks, waves.
+KSPLIT_TILES = ((1, 1, 8), (1, 2, 4), (2, 1, 4), (2, 2, 4), (1, 4, 4), (2, 4, 4), (4, 2, 4))
+# 16-bit groups of decode-sized M (<= 128) that run on the K-split kernel fuse at any
+# K while the weight holds at most this many elements (64 MB).  Measured (M x N x K,
+# bias + residual, fused and eager us a call): 1x1024x16384 13.5 and 30.7, 16x4096x4096
+# 10.8 and 28.2, 64x4096x8192 18.3 and 28.6, 128x1024x8192 13.4 and 28.7, 128x4096x8192
+# 24.5 and 37.2.  Larger weights are bound by memory on both paths and keep the rules
+# below (0.74-0.90 of eager up to 256 MB, 16x16384x16384 110.3 and 101.8).
+KSPLIT_MAX_WEIGHT = 1 << 25
+
+
+def runs_ksplit(M: int, N: int, K: int, cus: int = MI355X_CUS) -> bool:
+    """Whether the library runs a 16-bit M x N x K group on its K-split kernel
+    (choose_ksplit in csrc/gemm_epilogue.hip, both sides priced in us)."""
+    if K <= 0 or weight_streaming(M, N, cus) or (M > 128 and 2 * (-(-M // 256)) * (-(-N // 256)) > cus):
+        return False
+    least = float("inf")
+    for mb, nb, waves in KSPLIT_TILES:
+        tiles = -(-M // (16 * mb)) * -(-N // (16 * nb))
+        alone = waves * 2 * 16 * (mb + nb) * 128 > 80 * 1024  # one workgroup per CU
+        fixed = 5.1 if alone else 0.6 if mb * nb == 2 else 1.2
+        least = min(least, (1.0 if alone else 3.5) + max(1.0, tiles / cus) * (fixed + 0.32 * (mb + nb) * K / 1024))
+    tiled = -3.0 + partial_round_tile(M, N, K, cus)[1] / 160.0 * (5.05 + 3.6 * K / 1024)
+    return least < 0.85 * tiled
+
+
+def ksplit_beats_eager(M: int, N: int, K: int) -> bool:
+    """A 16-bit group of decode-sized M on the K-split kernel, KSPLIT_MAX_WEIGHT at most."""
+    return M <= 128 and N * K <= KSPLIT_MAX_WEIGHT and runs_ksplit(M, N, K)
+
 
 def weight_streaming(M: int, N: int, cus: int = MI355X_CUS) -> bool:
     """Decode-sized M against a wide weight: M <= 128 with at least one
@@ -222,12 +253,14 @@ def partial_round_tile(M: int, N: int, K: int, cus: int = MI355X_CUS) -> Tuple[T
     return best[0], best[1] / 5
 
 
-def few_tile_verdict(M: int, N: int, k_loop: int, min_tiles: int = MIN_TILES_LONG_K) -> Optional[str]:
+def few_tile_verdict(M: int, N: int, k_loop: int, min_tiles: int = MIN_TILES_LONG_K,
+                     ksplit: bool = True) -> Optional[str]:
     """Why a few-tile group stays eager (None: no objection): fewer than
     ``min_tiles`` 128x128 output tiles and a K loop of ``k_loop`` over more
-    than MAX_K_ROWS_PER_CU operand rows per CU."""
+    than MAX_K_ROWS_PER_CU operand rows per CU, unless the K-split kernel takes
+    it (``ksplit``: 16-bit operands) and beats eager."""
     tiles = -(-M // 128) * -(-N // 128)
-    if tiles >= min_tiles:
+    if tiles >= min_tiles or (ksplit and ksplit_beats_eager(M, N, k_loop)):
         return None
     (bm, bn), rows = partial_round_tile(M, N, k_loop)
     if k_loop * rows <= MAX_K_ROWS_PER_CU:
@@ -256,7 +289,8 @@ def trigger_is_fusible(node: torch.fx.Node, min_output_elements: int = MIN_FUSIO
         return False, f"tiny output {M}x{N}"
     if K % 8 != 0 and m1.dtype != torch.float32:  # the fp32 split pads K
         return False, f"K={K} is not a multiple of 8"
-    why = None if weight_streaming(M, N) else few_tile_verdict(M, N, effective_k(K, m1.dtype), min_tiles_long_k)
+    why = None if weight_streaming(M, N) else few_tile_verdict(
+        M, N, effective_k(K, m1.dtype), min_tiles_long_k, ksplit=m1.dtype != torch.float32)
     if why is not None:
         return False, f"K={K}, " + why
     return True, "fused"
@@ -361,7 +395,8 @@ def fused_beats_eager(spec: EpilogueSpec, K: int, k_per_pass: int = K_PER_EPILOG
     fp32 groups always fuse: eager runs an fp32 GEMM at the fp32 MFMA rate
     (157 TFLOP/s peak), the split product at a third of the bf16 rate.
     Weight-streaming shapes (``M`` and ``N`` given, :func:`weight_streaming`)
-    fuse while K <= WEIGHT_STREAM_K_PER_PASS x passes."""
+    fuse while K <= WEIGHT_STREAM_K_PER_PASS x passes, and those the K-split
+    kernel takes at every K (:func:`ksplit_beats_eager`)."""
     if k_per_pass <= 0 or dtype == torch.float32:
         return True, "fused"
     passes = epilogue_passes(spec, gemm_is_addmm)
@@ -370,6 +405,8 @@ def fused_beats_eager(spec: EpilogueSpec, K: int, k_per_pass: int = K_PER_EPILOG
             return True, "fused (decode-sized M: both paths stream the weight)"
         return False, (f"K={K} with {passes} elementwise pass(es) at decode-sized M: eager's GEMM streams "
                        f"the weight faster (fused iff K <= {WEIGHT_STREAM_K_PER_PASS} x passes)")
+    if M is not None and N is not None and ksplit_beats_eager(M, N, K):
+        return True, "fused (small output: the waves of a workgroup split K)"
     limit = k_per_pass * passes - k_offset
     if K <= limit:
         return True, "fused"

@@ -423,3 +423,30 @@ def test_output_aliasing_an_input_keeps_the_aot_wrapper(recorded):
     assert torch.allclose(y.float(), ry.float(), atol=1e-2)
     assert v.data_ptr() == x.data_ptr() and v.shape == (32 * 64,)  # still a view of the input
     assert be.dispatch and be.dispatch[0].startswith("aot: aliased outputs")
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1024, 16384), (16, 4096, 16384), (17, 1000, 4096), (64, 16384, 4096),
+                                   (64, 4096, 8192), (128, 32640, 256), (128, 32641, 256), (129, 256, 8192),
+                                   (512, 1024, 8192), (512, 2048, 4096), (1024, 1024, 1024), (2048, 1024, 4096),
+                                   (4096, 256, 256), (16384, 512, 1024)])
+def test_runs_ksplit_mirrors_the_library(M, N, K):
+    """compiler.runs_ksplit is the library's own choice (no device needed), and
+    a decode-sized group it takes fuses at every K up to KSPLIT_MAX_WEIGHT."""
+    import ctypes
+
+    from fuseml_amd import _abi
+    from fuseml_amd.epilogue import EpilogueSpec, EpiOp
+
+    d = _abi.GemmDesc()
+    d.M, d.N, d.K, d.ab_dtype = M, N, K, _abi.BF16
+    d.a, d.b, d.out.ptr = 0x10000, 0x20000, 0x30000
+    d.lda = d.ldb = K
+    d.out.ld, d.out.dtype = N, _abi.BF16
+    cfg = (ctypes.c_int32 * 4)()
+    got = _abi.load_library().fuseml_gemm_epilogue_ksplit(ctypes.byref(d), cfg)
+    assert got >= 0 and bool(got) == comp.runs_ksplit(M, N, K)
+    if got and M <= 128 and N * K <= comp.KSPLIT_MAX_WEIGHT:
+        spec = EpilogueSpec(1, 2, (EpiOp("add", 0), EpiOp("add", 3)), torch.bfloat16)
+        assert comp.few_tile_verdict(M, N, K) is None
+        assert comp.fused_beats_eager(spec, K, dtype=torch.bfloat16, M=M, N=N)[0]
+    assert not comp.ksplit_beats_eager(16, 16384, 16384)
