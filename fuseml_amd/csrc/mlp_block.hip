@@ -573,19 +573,20 @@ void mlp_block_kernel_isplit(const fuseml_mlp_desc d) {
 
 // The block with I split over eight waves, two per SIMD, in two groups that run
 // a super-chunk's phases in a different order, on packed weights (I a multiple of
-// 128; the last super-chunk is packed with zeros past I).  Super-chunk c holds 256 intermediate columns; wave w computes
-// h[rows, 32] of them (GEMM1 over all of D), adds b1, applies GELU and writes
-// them to the LDS h tile, and multiplies the whole h tile by its D/8 rows of W2
-// (GEMM2).  Between two barriers waves 0-3 run GEMM1(c), GELU(c), GEMM2(c - 1)
+// 128).  Super-chunk c holds 256 intermediate columns; wave w computes h[rows, 32]
+// of them (GEMM1 over all of D), adds b1, applies GELU and writes them to the LDS
+// h tile, and multiplies the whole h tile by its D/8 rows of W2 (GEMM2).  Where
+// the last super-chunk is half one (I an odd multiple of 128), its columns belong
+// to waves 0-3: waves 4-7 have no GEMM1 in it, and GEMM2 stops at its 128 columns.
+// (Zeros past I instead would turn an infinite x or h into NaN.)  Between two barriers waves 0-3 run GEMM1(c), GELU(c), GEMM2(c - 1)
 // and waves 4-7 GEMM2(c - 1), GEMM1(c), GELU(c): each SIMD holds one wave of
 // each group, so one wave's GELU (VALU) runs beside the other's MFMAs, where the
 // four-wave kernel above runs GEMM1, GELU and GEMM2 one after another on each
 // SIMD (20, 27 and 26% of its time at D = 256, I = 1024, for 26% of MFMA work).
 //   * h is double-buffered: step c writes h(c) and reads h(c - 1), and the buffer
 //     it writes was last read in step c - 1, a barrier earlier.
-//   * A wave's weight fragments lie in its order of consumption, 2 I / 256
-//     segments of D / 16 (fuseml_mlp_pack_weights), and stream through a ring of
-//     registers.
+//   * A wave's weight fragments lie in its order of consumption, segments of
+//     D / 16 (struct SkewPack), and stream through a ring of registers.
 //   * The MFMA loops of GEMM1 run at raised wave priority: the wave that feeds the
 //     other group's next phase is not held back by GELU instructions.
 // RB: 32-row blocks per workgroup.  Two where every CU gets 64 rows; one below
@@ -598,9 +599,26 @@ void mlp_block_kernel_isplit(const fuseml_mlp_desc d) {
 constexpr int kIS = 256;                    // intermediate columns per super-chunk
 constexpr int kSkewThreads = 512;
 
+// The packed weights of the kernel below: per wave a stream of 1 KB fragments, an
+// NS = D / 16 fragment segment for each GEMM1 (W1) and each GEMM2 (W2), with half a
+// segment for the GEMM2 of a half super-chunk, which waves 4-7 have no GEMM1 in.
+// 4 D I bytes in all.
+struct SkewPack {
+  int ns, nsc;   // fragments per segment, super-chunks
+  bool half;     // the last super-chunk is half one
+  __device__ SkewPack(int D, int I, bool half) : ns(D / 16), nsc((I + kIS - 1) / kIS), half(half) {}
+  __device__ int gemm1s(bool late) const { return nsc - (half && late ? 1 : 0); }
+  __device__ int frags(bool late) const { return (gemm1s(late) + nsc) * ns - (half ? ns / 2 : 0); }
+  __device__ int first(int wave) const {  // the wave's first fragment
+    return wave < 4 ? wave * frags(false) : 4 * frags(false) + (wave - 4) * frags(true);
+  }
+};
+
 __device__ __forceinline__ int hs_chunk(int m, int q) { return m * (kIS * 2) + ((q ^ (m & 15)) << 4); }
 
-template <int DW, int RB, int GELU, typename T>
+// HALF: the last super-chunk is half one.  A kernel of its own, since the conditions
+// in the loop cost the others 1-3% (13% at 1000; 512 -> 2048, 45.8 -> 51.7 us).
+template <int DW, int RB, int GELU, typename T, bool HALF>
 __global__ __launch_bounds__(kSkewThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void mlp_block_kernel_skew(const fuseml_mlp_desc d) {
   constexpr int D = 128 * DW;
@@ -624,12 +642,14 @@ void mlp_block_kernel_skew(const fuseml_mlp_desc d) {
   const bool late = wave >= 4;     // this wave's group runs GEMM2 first
   const int M = (int)d.M, I = (int)d.I;
   const int nblocks = (M + BM - 1) / BM;
-  const int nsc = (I + kIS - 1) / kIS;
+  const SkewPack pk(D, I, HALF);
+  const int nsc = pk.nsc;
+  const int gemm1s = pk.gemm1s(late);  // super-chunks with columns of this wave
 
   const __amdgpu_buffer_rsrc_t rb1 = make_rsrc(d.b1, (int64_t)I * 2);
-  // This wave's stream: 2 nsc segments of NS KB.
-  const int stream = 2 * nsc * NS * 1024;
-  const __amdgpu_buffer_rsrc_t rwp = make_rsrc(static_cast<const char*>(d.wpack) + (int64_t)wave * stream, stream);
+  const int stream = pk.frags(late) * 1024;
+  const __amdgpu_buffer_rsrc_t rwp =
+      make_rsrc(static_cast<const char*>(d.wpack) + (int64_t)pk.first(wave) * 1024, stream);
   const uint32_t wl = (uint32_t)(lane * 16);
   i32x4_t ring[RING];
 
@@ -651,8 +671,13 @@ void mlp_block_kernel_skew(const fuseml_mlp_desc d) {
                                                  0, 0, 0);
       }
     }
+    constexpr std::integral_constant<int, NS> kSegment;
     int pos = 0;  // byte offset of the current segment in the stream
-    static_for<0, RING>([&](auto f) { ring[f] = __builtin_amdgcn_raw_buffer_load_b128(rwp, wl, f * 1024, 0); });
+    static_for<0, RING>([&](auto f) {
+      // (half a segment, the whole stream at I = 128, can be shorter than the ring)
+      const int at = !HALF || f < NS / 2 || f * 1024 < stream ? f * 1024 : 0;
+      ring[f] = __builtin_amdgcn_raw_buffer_load_b128(rwp, wl, at, 0);
+    });
     f32x16_t acc[RB][DB];
     static_for<0, RB>([&](auto mb) {
       static_for<0, DB>([&](auto db) { static_for<0, 16>([&](auto r) { acc[mb][db][(int)r] = 0.0f; }); });
@@ -661,11 +686,12 @@ void mlp_block_kernel_skew(const fuseml_mlp_desc d) {
     barrier();  // x tile landed
 
     // Fragment f of the current segment, its slot refilled with the fragment
-    // RING further on (past the end of the stream: the first one, not used).
-    auto take = [&](auto f) {
+    // RING further on (past the end of the stream: the first one, not used).  The
+    // stream holds at least `sure` fragments from the segment's start on.
+    auto take = [&](auto f, auto sure) {
       const i32x4_t w = ring[f % RING];
       int next = pos + (f + RING) * 1024;
-      if constexpr (f + RING >= NS) next = next < stream ? next : 0;
+      if constexpr (f + RING >= sure) next = next < stream ? next : 0;
       ring[f % RING] = __builtin_amdgcn_raw_buffer_load_b128(rwp, wl, next, 0);
       return w;
     };
@@ -678,7 +704,7 @@ void mlp_block_kernel_skew(const fuseml_mlp_desc d) {
       static_for<0, RB>([&](auto mb) { static_for<0, 16>([&](auto r) { h1[mb][(int)r] = 0.0f; }); });
       __builtin_amdgcn_s_setprio(1);
       static_for<0, NS>([&](auto s) {
-        const i32x4_t w = take(s);
+        const i32x4_t w = take(s, kSegment);
         static_for<0, RB>([&](auto mb) {
           const int m = 32 * mb + l32;
           const i32x4_t xf = *reinterpret_cast<const i32x4_t*>(xs + x_chunk(m, 2 * s + kh, PITCH));
@@ -709,9 +735,10 @@ void mlp_block_kernel_skew(const fuseml_mlp_desc d) {
         });
       });
     };
-    auto gemm2 = [&](int c) {
+    // The h columns [16 B, 16 E) of super-chunk c.
+    auto gemm2_steps = [&](int c, auto b, auto e, auto sure) {
       const char* hb = hs + (c & 1) * kH;
-      static_for<0, kIS / 16>([&](auto s) {
+      static_for<decltype(b)::value, decltype(e)::value>([&](auto s) {
         i32x4_t hf[RB];
         static_for<0, RB>([&](auto mb) {
           const int m = 32 * mb + l32;
@@ -720,22 +747,31 @@ void mlp_block_kernel_skew(const fuseml_mlp_desc d) {
           hf[mb] = x;
         });
         static_for<0, DB>([&](auto db) {
-          const i32x4_t w = take(std::integral_constant<int, DB * decltype(s)::value + decltype(db)::value>{});
+          const i32x4_t w = take(std::integral_constant<int, DB * decltype(s)::value + decltype(db)::value>{}, sure);
           static_for<0, RB>([&](auto mb) { acc[mb][db] = mfma32<T>(w, hf[mb], acc[mb][db]); });
         });
       });
+    };
+    constexpr std::integral_constant<int, 0> kStep0;
+    constexpr std::integral_constant<int, kIS / 32> kStepHalf;
+    constexpr std::integral_constant<int, kIS / 16> kStepAll;
+    auto gemm2 = [&](int c) {
+      gemm2_steps(c, kStep0, kStepAll, kSegment);
       pos += NS * 1024;
     };
 
-    gemm1(0);
+    if (!HALF || gemm1s > 0) gemm1(0);
     barrier();
     for (int c = 1; c < nsc; ++c) {
       if (late) gemm2(c - 1);
-      gemm1(c);
+      if (!HALF || c < gemm1s) gemm1(c);
       if (!late) gemm2(c - 1);
       barrier();  // h(c) complete, h(c - 1) read
     }
-    gemm2(nsc - 1);
+    if constexpr (HALF)
+      gemm2_steps(nsc - 1, kStep0, kStepHalf, std::integral_constant<int, NS / 2>{});
+    else
+      gemm2(nsc - 1);
 
     // y = acc + b2 + r; acc[mb][db][r] is y[m0 + 32 mb + l32][wave D/8 + 32 db +
     // 8 (r>>2) + 4 kh + (r&3)].
@@ -778,37 +814,36 @@ void mlp_block_kernel_skew(const fuseml_mlp_desc d) {
   }
 }
 
-// fuseml_mlp_pack_weights, the order of the kernel above: block b is fragment f of segment q of
-// wave w's stream (b = (2 nsc w + q) NS + f).  Segment 0 is W1 of super-chunk 0;
-// then, per super-chunk c >= 1, W1(c) and W2(c - 1) for waves 0-3, W2(c - 1) and
-// W1(c) for waves 4-7; the last is W2 of the last super-chunk.
+// fuseml_mlp_pack_weights, one block per fragment of the order above.  Segment q of
+// waves 0-3: W1 of super-chunk 0, then W1(c) and W2(c - 1) per c >= 1, at last W2 of
+// the last super-chunk.  Of waves 4-7: W1(c) and W2(c) per super-chunk, without W1 of
+// a half one.
 __global__ __launch_bounds__(64) void mlp_pack_kernel(const fuseml_mlp_desc d, char* wpack) {
-  const int D = (int)d.D, NS = D / 16, DB = D / 256;
-  const int I = (int)d.I;
-  const int nsc = (I + kIS - 1) / kIS;
+  const int D = (int)d.D, DB = D / 256;
+  const SkewPack pk(D, (int)d.I, d.I % kIS != 0);
   const int b = blockIdx.x;
-  const int f = b % NS, q = (b / NS) % (2 * nsc), w = b / (2 * nsc * NS);
+  const bool late = b >= pk.first(4);
+  const int w = late ? 4 + (b - pk.first(4)) / pk.frags(true) : b / pk.frags(false);
+  const int t = b - pk.first(w), q = t / pk.ns, f = t % pk.ns;
   const int l32 = threadIdx.x & 31, kh = threadIdx.x >> 5;
-  const bool first = q == 0, last = q == 2 * nsc - 1;
-  const bool odd = (q & 1) != 0;                         // segments 2 c - 1, 2 c: step c
-  const bool is_w1 = first || (!last && (odd == (w < 4)));
-  const int step = (q + 1) / 2;                          // q = 2 c - 1 or 2 c -> c
-  // Rows of W1 and columns of W2 past I are zeros (I is a multiple of 128, so a
-  // fragment lies wholly on one side).
-  const uint16_t* src = nullptr;
-  if (is_w1) {
-    const int c = first ? 0 : step;
-    if (kIS * c + 32 * w < I)
-      src = static_cast<const uint16_t*>(d.w1) + (int64_t)(kIS * c + 32 * w + l32) * d.ldw1 + 16 * f + 8 * kh;
+  bool is_w1;
+  int c;
+  if (late) {
+    is_w1 = q < 2 * pk.gemm1s(true) && (q & 1) == 0;
+    c = q < 2 * pk.gemm1s(true) ? q / 2 : pk.nsc - 1;
   } else {
-    const int c = last ? nsc - 1 : step - 1;
-    const int s = f / DB, db = f % DB;
-    if (kIS * c + 16 * s < I)
-      src = static_cast<const uint16_t*>(d.w2) + (int64_t)(w * (D / 8) + 32 * db + l32) * d.ldw2 + kIS * c + 16 * s + 8 * kh;
+    const bool last = q == 2 * pk.nsc - 1;
+    is_w1 = q == 0 || (!last && (q & 1) != 0);
+    c = is_w1 ? (q + 1) / 2 : last ? pk.nsc - 1 : q / 2 - 1;
   }
-  i32x4_t x = {0, 0, 0, 0};
-  if (src != nullptr) x = *reinterpret_cast<const i32x4_t*>(src);
-  *reinterpret_cast<i32x4_t*>(wpack + (int64_t)b * 1024 + threadIdx.x * 16) = x;
+  const uint16_t* src;
+  if (is_w1) {
+    src = static_cast<const uint16_t*>(d.w1) + (int64_t)(kIS * c + 32 * w + l32) * d.ldw1 + 16 * f + 8 * kh;
+  } else {
+    const int s = f / DB, db = f % DB;
+    src = static_cast<const uint16_t*>(d.w2) + (int64_t)(w * (D / 8) + 32 * db + l32) * d.ldw2 + kIS * c + 16 * s + 8 * kh;
+  }
+  *reinterpret_cast<i32x4_t*>(wpack + (int64_t)b * 1024 + threadIdx.x * 16) = *reinterpret_cast<const i32x4_t*>(src);
 }
 
 void set_error(const char* msg) { fuseml_detail::set_error_text(msg); }
@@ -837,8 +872,8 @@ int device_cus(int dev) {
   return cus;
 }
 
-// Bytes of the packed weights: W1 and W2 with I rounded up to whole super-chunks.
-int64_t packed_bytes(const fuseml_mlp_desc& d) { return 4 * d.D * ((d.I + kIS - 1) / kIS * kIS); }
+// Bytes of the packed weights: W1 and W2.
+int64_t packed_bytes(const fuseml_mlp_desc& d) { return 4 * d.D * d.I; }
 
 int validate(const fuseml_mlp_desc* dp) {
   if (dp == nullptr) {
@@ -909,15 +944,20 @@ bool use_isplit(const fuseml_mlp_desc& d) {
   return d.I % kIC == 0 && d.D <= 512 && !force_dsplit;
 }
 
-template <int DW, int RB, typename T>
+template <int DW, int RB, typename T, bool HALF>
 hipError_t launch_skew(const fuseml_mlp_desc& d, int cus, hipStream_t s) {
   const int64_t blocks = (d.M + 32 * RB - 1) / (32 * RB);
   const dim3 grid((unsigned)(blocks < cus ? blocks : cus)), block(kSkewThreads);
   if (d.gelu == FUSEML_OP_GELU_TANH)
-    hipLaunchKernelGGL((mlp_block_kernel_skew<DW, RB, FUSEML_OP_GELU_TANH, T>), grid, block, 0, s, d);
+    hipLaunchKernelGGL((mlp_block_kernel_skew<DW, RB, FUSEML_OP_GELU_TANH, T, HALF>), grid, block, 0, s, d);
   else
-    hipLaunchKernelGGL((mlp_block_kernel_skew<DW, RB, FUSEML_OP_GELU_ERF, T>), grid, block, 0, s, d);
+    hipLaunchKernelGGL((mlp_block_kernel_skew<DW, RB, FUSEML_OP_GELU_ERF, T, HALF>), grid, block, 0, s, d);
   return hipGetLastError();
+}
+
+template <int DW, typename T, bool HALF>
+hipError_t launch_skew_rows(const fuseml_mlp_desc& d, int cus, hipStream_t s) {
+  return d.M <= 32 * (int64_t)cus ? launch_skew<DW, 1, T, HALF>(d, cus, s) : launch_skew<DW, 2, T, HALF>(d, cus, s);
 }
 
 template <int DW, typename T>
@@ -925,7 +965,7 @@ hipError_t launch_dw(const fuseml_mlp_desc& d, int cus, hipStream_t s) {
   const bool tanh_gelu = d.gelu == FUSEML_OP_GELU_TANH;
   if constexpr (DW <= 4) {
     if (d.wpack != nullptr && use_isplit(d))
-      return d.M <= 32 * (int64_t)cus ? launch_skew<DW, 1, T>(d, cus, s) : launch_skew<DW, 2, T>(d, cus, s);
+      return d.I % kIS == 0 ? launch_skew_rows<DW, T, false>(d, cus, s) : launch_skew_rows<DW, T, true>(d, cus, s);
   }
   const int64_t nblocks = (d.M + kBM - 1) / kBM;
   const int grid = (int)(nblocks < cus ? nblocks : cus);

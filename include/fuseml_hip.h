@@ -265,8 +265,8 @@ int fuseml_mlp_block(const fuseml_mlp_desc* desc, void* stream);
 /* 1 if fuseml_mlp_block accepts `desc`, 0 if not (reason in fuseml_last_error()). */
 int fuseml_mlp_block_supported(const fuseml_mlp_desc* desc);
 
-/* Bytes of the repacked weights for `desc` (W1 and W2 reordered: 4 * D * I, I
- * rounded up to a multiple of 256), or 0 if its shape does not stream weight fragments (D not 256 or 512, or I
+/* Bytes of the repacked weights for `desc` (4 * D * I: W1 and W2 reordered),
+ * or 0 if its shape does not stream weight fragments (D not 256 or 512, or I
  * not a multiple of 128).  Host only. */
 int64_t fuseml_mlp_pack_bytes(const fuseml_mlp_desc* desc);
 
@@ -274,9 +274,10 @@ int64_t fuseml_mlp_pack_bytes(const fuseml_mlp_desc* desc);
  * 16-byte aligned) in the order the single-kernel MLP consumes them: per wave,
  * each 16-byte-per-lane MFMA fragment as one contiguous 1 KB block, so every
  * fragment load is whole cache lines (read from W1 and W2 as they are, each lane
- * takes 32 bytes from each of 32 rows); zeros past I.  Asynchronous on `stream`.
- * The caller re-packs after changing W1 or W2.  No reference counterpart: the
- * reference has no single-kernel MLP. */
+ * takes 32 bytes from each of 32 rows).  Asynchronous on `stream`.  The order is the
+ * kernel's own: `wpack` serves the library that wrote it.  The caller re-packs after
+ * changing W1 or W2.  No reference counterpart: the reference has no single-kernel
+ * MLP. */
 int fuseml_mlp_pack_weights(const fuseml_mlp_desc* desc, void* wpack, void* stream);
 
 /* ------------------------------------------------------------------------
