@@ -125,14 +125,17 @@ class _Plan:
     plan on split operands.
 
     ``fast``: a call needs only the pointers (no negative strides, no operand
-    rebuilt per call, no fp32 split, a non-empty output), written through
-    ``words``, the descriptor as uint64 words; ``a_ok`` / ``b_ok``: the GEMM
-    operands' strides are K-major as the kernel reads them (their base
-    alignment is still checked per call)."""
+    rebuilt per call, no fp32 split, a non-empty output); ``a_ok`` / ``b_ok``:
+    the GEMM operands' strides are K-major as the kernel reads them (their base
+    alignment is still checked per call).
 
-    __slots__ = ("desc", "M", "N", "K", "neg", "operands", "nbytes", "k_split", "fast", "words", "desc_ref",
+    A call writes its pointers into a descriptor that is its own until the library
+    has read it (:meth:`take`: ``desc``, or a copy while another thread's call holds
+    that), so threads may share a plan."""
+
+    __slots__ = ("desc", "M", "N", "K", "neg", "operands", "nbytes", "k_split", "fast", "free", "desc_ref",
                  "a_ok", "b_ok", "lda", "ldb", "op_words", "red_words", "extra_words", "single_tile", "direct",
-                 "split_plan", "calls")
+                 "split_plan", "calls", "handed_over")
 
     def __init__(self) -> None:
         self.desc = _abi.GemmDesc()
@@ -144,8 +147,9 @@ class _Plan:
         self.operands: List[Tuple[int, bool]] = []  # (input index, rebuilt per call)
         self.nbytes: Optional[int] = None  # algorithmic bytes, for the timing hook
         self.fast = False
-        self.words = (ctypes.c_uint64 * (ctypes.sizeof(_abi.GemmDesc) // _WORD)).from_buffer(self.desc)
         self.desc_ref = ctypes.byref(self.desc)
+        # the descriptors that no call is using: as many as calls ran at once
+        self.free: List["_CallDesc"] = [_CallDesc(self.desc)]
         self.a_ok = self.b_ok = False
         self.lda = self.ldb = 0
         self.op_words: List[Tuple[int, int]] = []     # (descriptor word, input index)
@@ -155,6 +159,27 @@ class _Plan:
         self.direct = False
         self.split_plan: Optional["_Plan"] = None
         self.calls = 0  # fast calls made in Python
+        self.handed_over = False  # to the native caller, whether or not it took the plan
+
+    def take(self) -> "_CallDesc":
+        """A descriptor for one call, to be put back on ``free`` (both are single
+        list operations, which threads may interleave)."""
+        try:
+            return self.free.pop()
+        except IndexError:
+            # the fields that the holder of `desc` may be writing are written anew
+            return _CallDesc(_abi.GemmDesc.from_buffer_copy(self.desc))
+
+
+class _CallDesc:
+    """A descriptor, also as uint64 words."""
+
+    __slots__ = ("desc", "words", "ref")
+
+    def __init__(self, desc: _abi.GemmDesc) -> None:
+        self.desc = desc
+        self.words = (ctypes.c_uint64 * (ctypes.sizeof(_abi.GemmDesc) // _WORD)).from_buffer(self.desc)
+        self.ref = ctypes.byref(self.desc)
 
 
 class HipKernelLauncher:
@@ -308,8 +333,7 @@ class HipKernelLauncher:
         descriptor with the operands as they are."""
         if a.stride(1) != 1 or b.stride(0) != 1:
             return
-        probe = _abi.GemmDesc()
-        ctypes.memmove(ctypes.byref(probe), plan.desc_ref, ctypes.sizeof(probe))
+        probe = _abi.GemmDesc.from_buffer_copy(plan.desc)
         probe.K, probe.ab_dtype, probe.lda, probe.ldb = plan.K, _abi.F32, a.stride(0), b.stride(1)
         # any aligned addresses: the calls' own are checked per call
         probe.a = probe.b = probe.out.ptr = 1 << 12
@@ -333,8 +357,7 @@ class HipKernelLauncher:
                     for t in (inputs[i] for i in self._used))
         plan = self._plans.get(key)
         if plan is None:
-            plan = self._make_plan(inputs)
-            self._plans[key] = plan
+            plan = self._plans.setdefault(key, self._make_plan(inputs))
         if plan.direct and (inputs[self.spec.left].data_ptr() | inputs[self.spec.right].data_ptr()) % 16:
             if plan.split_plan is None:
                 plan.split_plan = self._make_plan(inputs, allow_direct=False)
@@ -344,7 +367,7 @@ class HipKernelLauncher:
         if plan.fast and self.timing_events is None and isinstance(self._lib, ctypes.CDLL):
             out = self._launch_fast(plan, inputs)
             plan.calls += 1
-            if plan.calls == _NATIVE_AFTER and plan.a_ok and plan.b_ok:
+            if plan.calls >= _NATIVE_AFTER and not plan.handed_over and plan.a_ok and plan.b_ok:
                 # While the GPU works on this call.
                 self._add_native(plan, inputs)
             return out
@@ -354,19 +377,23 @@ class HipKernelLauncher:
         """Hand a plan whose calls need only pointers to the native caller, unless
         its results are cast or viewed after the launch."""
         spec = self.spec
-        if spec.output_shapes or any(dt is not torch.float32 for dt in spec.reduce_dtypes):
-            return
-        with _native_lock:  # one per launcher: it holds the launch count
+        with _native_lock:  # once per plan; one caller per launcher: it holds the launch count
+            if plan.handed_over:
+                return
+            plan.handed_over = True
+            if spec.output_shapes or any(dt is not torch.float32 for dt in spec.reduce_dtypes):
+                return
             if self._native is None:
                 self._native = self._native_type(self._n_inputs, tuple(self._used), self._fallback_guard is not None)
                 self._native_call = self._native.call
-        plan.words[_W_LDA], plan.words[_W_LDB] = plan.lda, plan.ldb
+        desc = _abi.GemmDesc.from_buffer_copy(plan.desc)
+        desc.lda, desc.ldb = plan.lda, plan.ldb
         if plan.single_tile:
             outputs = (("t", 0),)
         else:
             outputs = tuple(("t", 0) if o[0] == "tile" else
                             ("r", spec.reductions.index(o[1])) if o[0] == "red" else ("e", o[1]) for o in spec.outputs)
-        self._native.add(inputs, plan.desc, _abi.entry_address(plan.direct), spec.left, spec.right,
+        self._native.add(inputs, desc, _abi.entry_address(plan.direct), spec.left, spec.right,
                          tuple([(slot, op[0]) for slot, op in enumerate(plan.operands)]),
                          spec.out_dtype if spec.store_tile else None, spec.extra_dtypes,
                          tuple([_abi.RED_SLOT[name] for name in spec.reductions]), outputs)
@@ -382,7 +409,8 @@ class HipKernelLauncher:
             raise _abi.FuseMLHipError(
                 _abi.EINVAL, f"inputs on {sorted({str(inputs[i].device) for i in self._used})}: "
                 "every tensor must be on the launch's GPU")
-        w = plan.words
+        call = plan.take()
+        w = call.words
         pa, pb = a.data_ptr(), b.data_ptr()
         if plan.a_ok and pa % 16 == 0:
             w[_W_LDA] = plan.lda
@@ -421,7 +449,8 @@ class HipKernelLauncher:
                 w[wi] = t.data_ptr()
                 reds[name] = t
         entry = self._lib.fuseml_gemm_epilogue_f32 if plan.direct else self._lib.fuseml_gemm_epilogue
-        rc = entry(plan.desc_ref, torch._C._cuda_getCurrentRawStream(dev))
+        rc = entry(call.ref, torch._C._cuda_getCurrentRawStream(dev))
+        plan.free.append(call)
         if rc != _abi.OK:
             raise _abi.FuseMLHipError(rc, _abi.last_error(self._lib))
         self._python_launches += 1
@@ -465,7 +494,8 @@ class HipKernelLauncher:
                     t.fill_(0.0 if name == "sum" else float("nan"))
             return self._assemble(tile, extras, reds)
 
-        d = plan.desc
+        call = plan.take()
+        d = call.desc
         stream = torch._C._cuda_getCurrentRawStream(dev.index) if dev.type == "cuda" else 0
         if plan.k_split:
             a, b = self._split_operands(plan, a, b, stream)
@@ -495,7 +525,8 @@ class HipKernelLauncher:
                 ev0, ev1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             ev0.record()
         entry = self._lib.fuseml_gemm_epilogue_f32 if plan.direct else self._lib.fuseml_gemm_epilogue
-        rc = entry(ctypes.byref(d), ctypes.c_void_p(stream))
+        rc = entry(call.ref, ctypes.c_void_p(stream))
+        plan.free.append(call)
         if rc != _abi.OK:
             raise _abi.FuseMLHipError(rc, _abi.last_error(self._lib))
         if timing is not None:

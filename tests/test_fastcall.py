@@ -169,6 +169,39 @@ def test_threads_and_streams_share_a_launcher():
 
 
 @gpu
+def test_threads_share_a_launcher_from_its_first_call():
+    """The same without a call made before: calls of the Python path, the plan's
+    handover and native calls run at once, two threads' rows off 16 bytes (copied
+    per call) under the others' signature."""
+    M, N, K = 64, 264, 128
+    b, _, wt = _args(M, N, K, device="cuda")
+    ins, want = [], []
+    for t in range(4):
+        rows = torch.zeros(M * (K + 8) + 8, dtype=BF, device="cuda")[3 * (t % 2):].as_strided((M, K), (K + 8, 1))
+        rows.copy_(torch.randn(M, K, generator=torch.Generator().manual_seed(t)).to(BF))
+        ins.append((b, rows, wt))
+        want.append(HipKernelLauncher(SPEC, 3)(b, rows.contiguous(), wt))
+    torch.cuda.synchronize()
+    for _ in range(20):
+        L, bad = HipKernelLauncher(SPEC, 3), []
+        start = threading.Barrier(4)
+
+        def work(t):
+            with torch.cuda.stream(torch.cuda.Stream()):
+                start.wait()
+                outs = [L(*ins[t]) for _ in range(12)]
+                torch.cuda.current_stream().synchronize()
+                bad.extend(t for o in outs if not torch.equal(o, want[t]))
+
+        threads = [threading.Thread(target=work, args=(t,)) for t in range(4)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not bad and len(L._plans) == 1
+
+
+@gpu
 def test_native_call_in_a_graph_replays():
     L = HipKernelLauncher(SPEC, 3)
     b, x, wt = _args(device="cuda")
