@@ -86,18 +86,48 @@ _WORD = 8
 _MW = {f: getattr(_abi.MlpDesc, f).offset // _WORD for f in ("x", "w1", "b1", "w2", "b2", "r", "y", "wpack")}
 
 
+class _CallDesc:
+    """A descriptor, also as uint64 words."""
+
+    __slots__ = ("desc", "words", "ref")
+
+    def __init__(self, desc: "_abi.MlpDesc") -> None:
+        self.desc = desc
+        self.words = (ctypes.c_uint64 * (ctypes.sizeof(_abi.MlpDesc) // _WORD)).from_buffer(desc)
+        self.ref = ctypes.byref(desc)
+
+
 class _MlpPlan:
     """What a call needs that depends only on its input signature: the
-    descriptor with every non-pointer field filled (written through ``words``,
-    the descriptor as uint64 words) and the packed-weight size (0: none)."""
+    descriptor with every non-pointer field filled and the packed-weight size
+    (0: none).  A call writes its pointers into a descriptor that is its own
+    until the library has read it (:meth:`take`), so threads may share a plan."""
 
-    __slots__ = ("desc", "words", "desc_ref", "M", "D", "dtype", "pack_bytes")
+    __slots__ = ("desc", "free", "M", "D", "dtype", "pack_bytes")
 
     def __init__(self, desc: "_abi.MlpDesc", M: int, D: int, dtype: torch.dtype, pack_bytes: int) -> None:
         self.desc = desc
-        self.words = (ctypes.c_uint64 * (ctypes.sizeof(_abi.MlpDesc) // _WORD)).from_buffer(desc)
-        self.desc_ref = ctypes.byref(desc)
+        self.free = [_CallDesc(desc)]
         self.M, self.D, self.dtype, self.pack_bytes = M, D, dtype, pack_bytes
+
+    def take(self) -> _CallDesc:
+        """A descriptor for one call, to be put back on ``free``."""
+        try:
+            return self.free.pop()
+        except IndexError:
+            return _CallDesc(_abi.MlpDesc.from_buffer_copy(self.desc))
+
+
+class _Pack:
+    """Packed weights: the buffer, what it was packed from, and the stream and
+    event after which it is complete."""
+
+    __slots__ = ("key", "buf", "storages", "stream", "event", "complete")
+
+    def __init__(self, key: tuple, buf: torch.Tensor, storages: tuple, stream: int, event: Any) -> None:
+        # The storages are kept: while they live no other weight has their addresses.
+        self.key, self.buf, self.storages, self.stream, self.event = key, buf, storages, stream, event
+        self.complete = False
 
 
 class HipMlpLauncher:
@@ -117,16 +147,15 @@ class HipMlpLauncher:
         # Where the kernel streams weight fragments (D of 256 or 512, I a
         # multiple of 128), W1 and W2 are repacked once into fragment order
         # (fuseml_mlp_pack_weights: 4*D*I extra bytes, held here) and packed
-        # again when either weight changes (pointer, stride or in-place version).
+        # again when either weight changes (pointer, stride or in-place version;
+        # see repack for a change that none of them shows).
         self.pack_weights = pack_weights
-        self._pack: Optional[torch.Tensor] = None
-        self._pack_key: Optional[tuple] = None
+        self._pack: Optional[_Pack] = None
         # Per input signature (shapes, strides, dtypes, device): a plan whose
         # calls only write pointers (see launch).
         self._plans: Dict[tuple, _MlpPlan] = {}
         self._gelu = _abi.OP_GELU_TANH if approximate == "tanh" else _abi.OP_GELU_ERF
         self._lib = _abi.load_library()
-        self._desc = _abi.MlpDesc()
         self._guard = EagerFallbackGuard(eager_fn, kernel_signature) if eager_fn is not None else None
         self.launch_count = 0
 
@@ -151,18 +180,17 @@ class HipMlpLauncher:
             plan = self._plans.get(key)
             if plan is not None:
                 return self._launch_planned(plan, key, x, w1t, b1, w2t, b2, r)
-            y = self._launch_checked(x, w1t, b1, w2t, b2, r)
-            if self._plan_ok:
-                d = _abi.MlpDesc()
-                ctypes.memmove(ctypes.byref(d), ctypes.byref(self._desc), ctypes.sizeof(d))
-                self._plans[key] = _MlpPlan(d, int(x.shape[0]), int(x.shape[1]), x.dtype, self._plan_pack_bytes)
+            y, plan = self._launch_checked(x, w1t, b1, w2t, b2, r)
+            if plan is not None:
+                self._plans.setdefault(key, plan)
             return y
-        return self._launch_checked(x, w1t, b1, w2t, b2, r)
+        return self._launch_checked(x, w1t, b1, w2t, b2, r)[0]
 
     def _launch_planned(self, plan: "_MlpPlan", key: tuple, x: torch.Tensor, w1t: torch.Tensor,
                         b1: torch.Tensor, w2t: torch.Tensor, b2: Optional[torch.Tensor],
                         r: Optional[torch.Tensor]) -> torch.Tensor:
-        w = plan.words
+        call = plan.take()
+        w = call.words
         w[_MW["x"]] = x.data_ptr()
         w[_MW["w1"]] = w1t.data_ptr()
         w[_MW["b1"]] = b1.data_ptr()
@@ -172,32 +200,57 @@ class HipMlpLauncher:
         y = torch.empty((plan.M, plan.D), dtype=plan.dtype, device=x.device)
         w[_MW["y"]] = y.data_ptr()
         stream = torch._C._cuda_getCurrentRawStream(x.get_device())
-        w[_MW["wpack"]] = self._packed(plan.desc_ref, plan.pack_bytes, x, w1t, w2t, stream) if plan.pack_bytes else 0
-        rc = self._lib.fuseml_mlp_block(plan.desc_ref, ctypes.c_void_p(stream))
+        w[_MW["wpack"]] = 0
+        if plan.pack_bytes:
+            pack = self._packed(call.ref, plan.pack_bytes, x, w1t, w2t, stream)  # alive until the launch is queued
+            w[_MW["wpack"]] = pack.data_ptr()
+        rc = self._lib.fuseml_mlp_block(call.ref, ctypes.c_void_p(stream))
+        plan.free.append(call)
         if rc != _abi.OK:
             raise _abi.FuseMLHipError(rc, _abi.last_error(self._lib))
         self.launch_count += 1
         return y
 
     def _packed(self, desc_ref: Any, nbytes: int, x: torch.Tensor, w1t: torch.Tensor, w2t: torch.Tensor,
-                stream: int) -> int:
-        """The packed weights' address (packed again when W1 or W2 changed)."""
-        key = (x.device, nbytes, w1t.data_ptr(), w1t.stride(1), w1t._version, w2t.data_ptr(), w2t.stride(1),
+                stream: int) -> torch.Tensor:
+        """The packed weights (packed again when W1 or W2, as the caller passed
+        them, changed), ready for the current stream `stream`."""
+        key = (x.device, nbytes, w1t.data_ptr(), w1t.stride(), w1t._version, w2t.data_ptr(), w2t.stride(),
                w2t._version)
-        if key != self._pack_key:
+        pack = self._pack
+        if pack is None or pack.key != key:
             buf = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
             rc = self._lib.fuseml_mlp_pack_weights(desc_ref, ctypes.c_void_p(buf.data_ptr()), ctypes.c_void_p(stream))
             if rc != _abi.OK:
                 raise _abi.FuseMLHipError(rc, _abi.last_error(self._lib))
-            self._pack, self._pack_key = buf, key
-        return self._pack.data_ptr()
+            if not torch.cuda.is_current_stream_capturing():
+                # (packed while a graph is captured, it is filled by that graph's replays alone)
+                event = torch.cuda.Event()
+                event.record(torch.cuda.current_stream(x.device))
+                self._pack = _Pack(key, buf, (w1t.untyped_storage(), w2t.untyped_storage()), stream, event)
+            return buf
+        if stream != pack.stream and not torch.cuda.is_current_stream_capturing():
+            # Another stream than the one it was packed on (a capture starts after
+            # the work before it, and takes neither a wait nor a query).
+            current = torch.cuda.current_stream(x.device)
+            if not pack.complete:
+                if pack.event.query():
+                    pack.complete = True
+                else:
+                    current.wait_event(pack.event)
+            pack.buf.record_stream(current)  # a later repack frees it behind this call
+        return pack.buf
+
+    def repack(self) -> None:
+        """Have the next call pack the weights anew: after a change that leaves
+        their address and version alone (a write through ``weight.data``)."""
+        self._pack = None
 
     def _launch_checked(self, x: torch.Tensor, w1t: torch.Tensor, b1: torch.Tensor, w2t: torch.Tensor,
-                        b2: Optional[torch.Tensor], r: Optional[torch.Tensor]) -> torch.Tensor:
-        # whether this call's descriptor may serve later calls of its signature
-        # (operands used in place, not copied), and its packed-weight size
-        self._plan_ok = False
-        self._plan_pack_bytes = 0
+                        b2: Optional[torch.Tensor],
+                        r: Optional[torch.Tensor]) -> Tuple[torch.Tensor, Optional[_MlpPlan]]:
+        """The result, and a plan for later calls of this signature where the
+        operands were used in place."""
         if x.dim() != 2 or w1t.dim() != 2 or w2t.dim() != 2:
             raise _abi.FuseMLHipError(_abi.EUNSUPPORTED, "mlp_block takes 2-D x and weights")
         M, D = x.shape
@@ -216,6 +269,7 @@ class HipMlpLauncher:
         # K-contiguous operands (the graph's layouts: x row-major, t(W) views).
         in_place = (x.stride(1) == 1 and w1t.stride(0) == 1 and w2t.stride(0) == 1 and b1.is_contiguous()
                     and (b2 is None or b2.is_contiguous()) and (r is None or r.stride(1) == 1))
+        weights = w1t, w2t
         if x.stride(1) != 1:
             x = x.contiguous()
         if w1t.stride(0) != 1:
@@ -229,8 +283,8 @@ class HipMlpLauncher:
             r = r.contiguous()
         y = torch.empty((M, D), dtype=dt, device=x.device)
         if M == 0:
-            return y
-        d = self._desc
+            return y, None
+        d = _abi.MlpDesc()
         d.M, d.D, d.I = M, D, I
         d.x, d.ldx = x.data_ptr(), x.stride(0)
         d.w1, d.ldw1 = w1t.data_ptr(), w1t.stride(1)
@@ -250,13 +304,13 @@ class HipMlpLauncher:
         if self.pack_weights and isinstance(self._lib, ctypes.CDLL):
             nbytes = self._lib.fuseml_mlp_pack_bytes(ctypes.byref(d))
             if nbytes > 0:
-                d.wpack = self._packed(ctypes.byref(d), nbytes, x, w1t, w2t, stream)
+                pack = self._packed(ctypes.byref(d), nbytes, x, *weights, stream)  # alive until the launch is queued
+                d.wpack = pack.data_ptr()
         rc = self._lib.fuseml_mlp_block(ctypes.byref(d), ctypes.c_void_p(stream))
         if rc != _abi.OK:
             raise _abi.FuseMLHipError(rc, _abi.last_error(self._lib))
         self.launch_count += 1
-        self._plan_ok, self._plan_pack_bytes = in_place, nbytes
-        return y
+        return y, _MlpPlan(d, M, D, dt, nbytes) if in_place else None
 
     def __call__(self, *inputs: Any) -> torch.Tensor:
         if len(inputs) != self.N_INPUTS:
