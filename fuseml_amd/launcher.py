@@ -223,6 +223,10 @@ class HipKernelLauncher:
     def launch_count(self) -> int:
         return self._python_launches + (self._native.count if self._native is not None else 0)
 
+    @launch_count.setter
+    def launch_count(self, value: int) -> None:
+        self._python_launches = value - (self._native.count if self._native is not None else 0)
+
     @property
     def fallback_count(self) -> int:
         return self._fallback_guard.fallback_count if self._fallback_guard else 0

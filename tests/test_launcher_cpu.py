@@ -370,3 +370,23 @@ def test_fp32_plan_is_direct_only_for_k_major_aligned_operands(make_x, make_wt, 
     assert plan.desc.ab_dtype == (_abi.F32 if direct else _abi.BF16)
     big = launcher._make_plan((torch.randn(4096, K), torch.randn(2048, K).t()))  # a large output: split passes
     assert not big.direct and big.k_split == K
+
+
+def test_launch_count_can_be_set():
+    """A caller may reset the count, with launches of either path behind it."""
+    rec = Recorder()
+    launcher = make(EpilogueSpec(0, 1, (EpiOp("relu"),), BF), 2, rec)
+    args = torch.randn(8, 16, dtype=BF), torch.randn(8, 16, dtype=BF).t()
+
+    class Native:
+        count = 5
+
+    launcher(*args)
+    assert launcher.launch_count == 1
+    launcher._native = Native()
+    assert launcher.launch_count == 6
+    launcher.launch_count = 0
+    assert launcher.launch_count == 0
+    Native.count += 2
+    launcher(*args)
+    assert launcher.launch_count == 3
