@@ -23,7 +23,9 @@ kernel_launcher.py:496-509, 816-821, extended to sum and amax).
 from __future__ import annotations
 
 import ctypes
+import functools
 import threading
+import warnings
 from typing import Any, Callable, Dict, List, Optional, Sequence, Tuple
 
 import torch
@@ -111,6 +113,17 @@ assert all(o % _WORD == 0 for o in (_abi.GemmDesc.a.offset, _abi.GemmDesc.operan
 # signature that is seen once or twice would not get back.
 _NATIVE_AFTER = 3
 _native_lock = threading.Lock()
+
+
+@functools.lru_cache(maxsize=None)
+def _native_type() -> Optional[type]:
+    """The native caller's type, or None with a warning where the extension is not
+    built, or built for another Python or torch: Python serves every call then."""
+    try:
+        return _abi.load_fastcall()
+    except ImportError as exc:
+        warnings.warn(f"repeated launches stay in Python: {exc}", RuntimeWarning)
+        return None
 
 
 class _Plan:
@@ -214,7 +227,7 @@ class HipKernelLauncher:
         self._used = sorted({spec.left, spec.right} | {op.operand for op in spec.ops if op.kind in ("add", "mul")})
         # Repeated calls of a signature whose plan needs only pointers run in native
         # code (csrc/fastcall.cpp); it declines every other call.
-        self._native_type = _abi.load_fastcall()
+        self._native_type = _native_type()
         self._native: Optional[Any] = None  # made with the first plan handed over
         self._native_call: Optional[Callable[..., Any]] = None
 
@@ -385,7 +398,7 @@ class HipKernelLauncher:
             if plan.handed_over:
                 return
             plan.handed_over = True
-            if spec.output_shapes or any(dt is not torch.float32 for dt in spec.reduce_dtypes):
+            if self._native_type is None or spec.output_shapes or any(dt is not torch.float32 for dt in spec.reduce_dtypes):
                 return
             if self._native is None:
                 self._native = self._native_type(self._n_inputs, tuple(self._used), self._fallback_guard is not None)

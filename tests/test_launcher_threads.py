@@ -7,11 +7,12 @@ from __future__ import annotations
 
 import ctypes
 import threading
+import warnings
 
 import pytest
 import torch
 
-from fuseml_amd import _abi
+from fuseml_amd import _abi, launcher
 from fuseml_amd.epilogue import EpilogueSpec, EpiOp
 from fuseml_amd.launcher import _NATIVE_AFTER, HipKernelLauncher
 
@@ -133,3 +134,24 @@ def test_a_plan_is_handed_over_past_its_due_call(on_a_device):
     for _ in range(3):
         L(*args)
     assert len(Native.plans) == 1
+
+
+def test_calls_without_the_native_caller(on_a_device, monkeypatch):
+    """Where the extension is missing, Python serves every call, with one warning."""
+    def missing():
+        raise ImportError("no extension")
+
+    monkeypatch.setattr(_abi, "load_fastcall", missing)
+    launcher._native_type.cache_clear()
+    try:
+        with pytest.warns(RuntimeWarning, match="no extension"):
+            L = HipKernelLauncher(SPEC, 3)
+        with warnings.catch_warnings():
+            warnings.simplefilter("error")
+            HipKernelLauncher(SPEC, 3)
+    finally:
+        launcher._native_type.cache_clear()
+    L._lib = Library()
+    for _ in range(_NATIVE_AFTER + 2):
+        L(*_args())
+    assert L.launch_count == _NATIVE_AFTER + 2 and L._native is None
