@@ -273,8 +273,9 @@ def entry_address(f32: bool) -> int:
     loaded library, for the native caller."""
     if not _entries:
         lib = load_library()
-        for key, fn in ((False, lib.fuseml_gemm_epilogue), (True, lib.fuseml_gemm_epilogue_f32)):
-            _entries[key] = ctypes.cast(fn, ctypes.c_void_p).value
+        fns = {False: lib.fuseml_gemm_epilogue, True: lib.fuseml_gemm_epilogue_f32}
+        # both at once: another thread finds none or both
+        _entries.update({key: ctypes.cast(fn, ctypes.c_void_p).value for key, fn in fns.items()})
     return _entries[f32]
 
 

@@ -155,3 +155,19 @@ def test_calls_without_the_native_caller(on_a_device, monkeypatch):
     for _ in range(_NATIVE_AFTER + 2):
         L(*_args())
     assert L.launch_count == _NATIVE_AFTER + 2 and L._native is None
+
+
+def test_entry_addresses_appear_together(monkeypatch):
+    """Another thread that asks while they are looked up finds none or both."""
+    monkeypatch.setattr(_abi, "_entries", {})
+    cast, others = ctypes.cast, []
+
+    def casting(fn, kind):
+        if _abi._entries and not others:
+            others.append(None)
+            others[0] = _abi.entry_address(True)
+        return cast(fn, kind)
+
+    monkeypatch.setattr(_abi.ctypes, "cast", casting)
+    want = _abi.entry_address(False), _abi.entry_address(True)
+    assert all(want) and want[0] != want[1] and set(others) <= {want[1]}
