@@ -188,7 +188,7 @@ def _gemm_dims(group: Any) -> Tuple[Optional[int], Any, Optional[int], Optional[
 # eager's time at K = 2048-4096, 1.07 at K = 8192).
 WEIGHT_STREAM_K_PER_PASS = 4096
 
-# The library's K-split tiles (kKsplit in csrc/gemm_epilogue_shared.h): 16-row and
+# The library's K-split tiles (kKsplit in csrc/ksplit_rule.h): 16-row and
 # 16-column blocks, waves.
 KSPLIT_TILES = ((1, 1, 8), (1, 2, 4), (2, 1, 4), (2, 2, 4), (1, 4, 4), (2, 4, 4), (4, 2, 4))
 # 16-bit groups of decode-sized M (<= 128) that run on the K-split kernel fuse at any

@@ -209,54 +209,18 @@ TileConfig choose_config(const fuseml_gemm_desc& d, int cus) {
 // Not at 1024x1024x1024 (11.0 tiled, 13.0 here: operands shared by more waves
 // win) nor where the weight streams through a full row of tiles
 // (16x65536x1024 28.5 against 30.7).
-//
-// cheapest_ksplit: the K-split tile with the least priced time, `per_k` us per
-// block row or column and 1024 of K.
-int cheapest_ksplit(const fuseml_gemm_desc& d, int cus, double per_k, double* least) {
-  int best = -1;
-  for (int i = 0; i < kNumKsplit; ++i) {
-    const KsplitConfig& c = kKsplit[i];
-    const double tiles = (double)(cdiv(d.M, c.bm()) * cdiv(d.N, c.bn()));
-    const double r = tiles > cus ? tiles / cus : 1.0;
-    const bool alone = c.lds_bytes() > 80 * 1024;
-    const double fixed = alone ? 5.1 : c.mb * c.nb == 2 ? 0.6 : 1.2;
-    const double t = (alone ? 1.0 : 3.5) + r * (fixed + per_k * (c.mb + c.nb) * (double)d.K / 1024.0);
-    if (best < 0 || t < *least) {
-      best = i;
-      *least = t;
-    }
-  }
-  return best;
-}
-
 int choose_ksplit(const fuseml_gemm_desc& d, int cus) {
   if (forced_variant() != 0 || d.K <= 0 || weight_streaming(d, cus)) return -1;
   if (d.M > 128 && 2 * cdiv(d.M, 256) * cdiv(d.N, 256) > cus) return -1;
   double cost = 0.0;
-  const int best = cheapest_ksplit(d, cus, 0.32, &cost);
+  const int best = cheapest_ksplit(d.M, d.N, d.K, cus, 0.32, &cost);
   int64_t work = 0;
   choose_partial_round(d, cus, &work);
   const double tiled = -3.0 + (double)work / (5.0 * 160.0) * (5.05 + 3.6 * (double)d.K / 1024.0);
   return cost < 0.85 * tiled ? best : -1;
 }
 
-// The K-split tile for fp32 GEMM operands, or -1 where splitting them into bf16
-// parts first (fuseml_split_bf16x3, three launches, 10 bytes of traffic per
-// element before the GEMM) is the faster way.  The K-split kernel reads 4 bytes
-// per element once and splits each fragment in registers, but every tile splits
-// its rows anew, at about 0.9 us per block and 1024 of K: it wins while the
-// output is small.  Measured (M x N x K, us, split passes and GEMM -> this):
-// 64x2048x512 15.9 -> 6.3, 1024x1024x1024 31 -> 22, 1024x1024x4096 80 -> 64,
-// 512x4096x256 23.8 -> 21.9, a tie at 2048x1024x1024 (38.0 and 39.0), and
-// 2048x2048x512 38.3 -> 52.7 the other way.
-int choose_ksplit_f32(const fuseml_gemm_desc& d, int cus) {
-  if (d.K <= 0) return -1;
-  double cost = 0.0;
-  const int best = cheapest_ksplit(d, cus, 0.9, &cost);
-  const KsplitConfig& c = kKsplit[best];
-  const int64_t padded = cdiv(d.M, c.bm()) * c.bm() * cdiv(d.N, c.bn()) * c.bn();
-  return d.M <= 32 || padded <= ((int64_t)1 << (d.K <= 512 ? 21 : 20)) ? best : -1;
-}
+int choose_ksplit_f32(const fuseml_gemm_desc& d, int cus) { return ksplit_f32(d.M, d.N, d.K, cus); }
 
 bool check_output(const fuseml_output& o, const fuseml_gemm_desc& d, const char* what) {
   if (o.ptr == nullptr) return true;
@@ -639,7 +603,7 @@ bool split_rounds(fuseml_gemm_desc& d, int cus, fuseml_gemm_desc& rest) {
   double small = 0.0;
   int64_t work = 0;
   choose_partial_round(r, cus, &work);
-  cheapest_ksplit(r, cus, 0.32, &small);
+  cheapest_ksplit(r.M, r.N, r.K, cus, 0.32, &small);
   const double tiled = -3.0 + (double)work / (5.0 * 160.0) * (5.05 + 3.6 * k);
   if (small >= 0.85 * tiled) small = tiled;
   if (small + 2.0 > 0.9 * partial) return false;

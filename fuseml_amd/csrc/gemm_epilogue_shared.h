@@ -10,6 +10,7 @@
 #include <stdint.h>
 
 #include "fuseml_hip.h"
+#include "ksplit_rule.h"
 
 namespace fuseml_gemm {
 
@@ -36,22 +37,6 @@ constexpr TileConfig kNarrow64 = {64, 128, 64, 3, 2, 2, 0};  // 4 waves lock-ste
 constexpr TileConfig kNarrow32 = {32, 128, 64, 3, 1, 4, 0};  // 4 waves lock-step (wave tile 32x32), 62 KB LDS, 2 WG/CU
 constexpr TileConfig kLarge128 = {256, 128, 32, 4, 4, 2, 1};  // 8 waves ping-pong (wave tile 64x64), 100 KB LDS, 1 WG/CU
 constexpr TileConfig kSmall64 = {128, 128, 64, 4, 2, 2, 0};  // kSmall at BK = 64: 130 KB LDS, 1 WG/CU
-
-// Tiles of the K-split kernel (gemm_ksplit.h): mb x nb blocks of 16 x 16, waves
-// splitting K, chunks of 128 bytes per row that a wave's LDS ring holds.
-struct KsplitConfig {
-  int mb, nb, waves, depth;
-  constexpr int bm() const { return 16 * mb; }
-  constexpr int bn() const { return 16 * nb; }
-  constexpr int lds_bytes() const {
-    const int ring = waves * depth * (bm() + bn()) * 128, part = waves * bm() * bn() * 4;
-    return ring > part ? ring : part;
-  }
-};
-
-constexpr KsplitConfig kKsplit[] = {{1, 1, 8, 2}, {1, 2, 4, 2}, {2, 1, 4, 2}, {2, 2, 4, 2},
-                                    {1, 4, 4, 2}, {2, 4, 4, 2}, {4, 2, 4, 2}};
-constexpr int kNumKsplit = 7;
 
 // Launch tile `index` of kKsplit; T: __bf16, _Float16 or float GEMM operands
 // (gemm_ksplit_v_*.hip).
