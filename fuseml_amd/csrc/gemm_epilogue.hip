@@ -441,26 +441,44 @@ int match_fixed_chain(const fuseml_gemm_desc& d) {
 
 // `max_wg` caps the grid (0: one workgroup per tile); the kernel loops over the
 // remaining tiles.
-template <const TileConfig& C>
-hipError_t launch_variant(const fuseml_gemm_desc& d, hipStream_t stream, int max_wg) {
+template <const TileConfig& C, bool ANY>
+hipError_t launch_rows(const fuseml_gemm_desc& d, hipStream_t stream, int max_wg) {
   int64_t tiles = cdiv(d.M, C.bm) * cdiv(d.N, C.bn);
   if (max_wg > 0 && tiles > max_wg) tiles = max_wg;
   const dim3 grid((unsigned)tiles), block(C.wm * C.wn * 64);
   const bool red = d.reduce_mask != 0;
   constexpr int G = kChainGeneric;
   if (d.ab_dtype == FUSEML_BF16 && !red)
-    hipLaunchKernelGGL((gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, C.sched, __bf16, false, G>),
+    hipLaunchKernelGGL((gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, C.sched, __bf16, false, G, ANY>),
                        grid, block, 0, stream, d);
   else if (d.ab_dtype == FUSEML_BF16)
-    hipLaunchKernelGGL((gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, C.sched, __bf16, true, G>),
+    hipLaunchKernelGGL((gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, C.sched, __bf16, true, G, ANY>),
                        grid, block, 0, stream, d);
   else if (!red)
-    hipLaunchKernelGGL((gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, C.sched, _Float16, false, G>),
+    hipLaunchKernelGGL((gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, C.sched, _Float16, false, G, ANY>),
                        grid, block, 0, stream, d);
   else
-    hipLaunchKernelGGL((gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, C.sched, _Float16, true, G>),
+    hipLaunchKernelGGL((gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, C.sched, _Float16, true, G, ANY>),
                        grid, block, 0, stream, d);
   return hipGetLastError();
+}
+
+// Whether a launch needs the kernel's parameter ANY: a staged operand whose rows are
+// not whole 16-byte chunks at 16-byte addresses, or an output that is not staged or
+// has such rows.
+bool needs_any(const fuseml_gemm_desc& d) {
+  constexpr int kBoth = kFlagStage | kFlagAligned;
+  for (int i = 0; i < d.n_operands; ++i)
+    if ((d.operands[i].reserved & kBoth) == kFlagStage) return true;
+  return d.out.ptr != nullptr && (d.out.reserved & kBoth) != kBoth;
+}
+
+template <const TileConfig& C>
+hipError_t launch_variant(const fuseml_gemm_desc& d, hipStream_t stream, int max_wg) {
+  if constexpr (splits_rows(C)) {
+    if (!needs_any(d)) return launch_rows<C, false>(d, stream, max_wg);
+  }
+  return launch_rows<C, true>(d, stream, max_wg);
 }
 
 // A fixed-chain kernel of variant C (reductions only with kChainRelu, as
@@ -469,12 +487,12 @@ template <const TileConfig& C, typename T, int CH>
 void launch_fixed_one(const fuseml_gemm_desc& d, hipStream_t stream, dim3 grid, dim3 block) {
   if constexpr (CH == kChainRelu) {
     if (d.reduce_mask != 0) {
-      hipLaunchKernelGGL((gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, C.sched, T, true, CH>), grid,
+      hipLaunchKernelGGL((gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, C.sched, T, true, CH, true>), grid,
                          block, 0, stream, d);
       return;
     }
   }
-  hipLaunchKernelGGL((gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, C.sched, T, false, CH>), grid,
+  hipLaunchKernelGGL((gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, C.sched, T, false, CH, true>), grid,
                      block, 0, stream, d);
 }
 

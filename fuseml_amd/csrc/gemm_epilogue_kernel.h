@@ -544,7 +544,11 @@ __device__ __forceinline__ i32x4_t swap_halves(i32x4_t x) { return i32x4_t{x.z, 
 // chain is the same arithmetic compiled as straight-line code (bitwise the
 // same results), which at one wave per SIMD removes the op loop's per-op
 // descriptor loads, dispatch and register copies from every column block.
-template <int BM, int BN, int BK, int S, int WM, int WN, int SCHED, typename T, bool RED, int CH>
+// ANY: staged rows may have any length and alignment, and the output need not be
+// staged.  Without it every staged operand has kFlagAligned and the output, where
+// there is one, kFlagStage and kFlagAligned (the host sees to it: needs_any), and the
+// kernel carries none of the code for the others.
+template <int BM, int BN, int BK, int S, int WM, int WN, int SCHED, typename T, bool RED, int CH, bool ANY>
 __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(SCHED >= 3 ? 1 : 2)))
 void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
   using G = StageGeom<BK>;
@@ -594,12 +598,16 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
     // kernels of the one-wave schedules also wait for the previous tile's
     // global stores: without that wait, the compiler's wait insertion sees
     // them as possibly pending at this tile's K loop and puts an s_waitcnt
-    // vmcnt(0) into the steady loop.  The other kernels leave the stores in
+    // vmcnt(0) into the steady loop.  So do the lock-step kernels, which have one
+    // tile per workgroup and nothing to wait for: else the compiler sees the
+    // epilogue's loads as pending in registers that the prologue writes, and waits
+    // for the row vectors' loads before the first DMA (2048x1024x4096 bias+residual
+    // 28.90 -> 28.65 us).  The other kernels leave the stores in
     // flight: their K loops' counted waits only get stricter for older
     // operations (vector-memory operations complete in issue order).
     __builtin_amdgcn_sched_barrier(0);
     wait_lgkmcnt0();
-    if constexpr (SCHED == 3 || (SCHED == 6 && CH == kChainGeneric)) wait_vmcnt<0>();
+    if constexpr (SCHED == 0 || SCHED == 3 || (SCHED == 6 && CH == kChainGeneric)) wait_vmcnt<0>();
     __builtin_amdgcn_sched_barrier(0);
     if (tile != (int)blockIdx.x) {
       asm volatile("" ::: "memory");
@@ -702,7 +710,7 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
     constexpr int RPS = STAGE / SP;   // staging rows per pipeline slot
     static_assert(!kOpDma || (STAGE % SP == 0 && RPS % 32 == 0 && RPS == RPD * NW * LPS),
                   "operand DMAs line up with the stage DMAs");
-    const bool staged_aligned = (staged_flags & kFlagAligned) != 0;
+    const bool staged_aligned = ANY ? (staged_flags & kFlagAligned) != 0 : staged >= 0;
     const bool op_dma = kOpDma && staged_aligned;
     const void* op_ptr = d.a;
     int64_t op_bytes = 0;  // bytes of the operand from its row m0 on
@@ -1284,7 +1292,7 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
       constexpr int NP = BM / RPP;
       constexpr int PB = NP < 8 ? NP : 8;
       static_assert(NP % PB == 0, "pass batches");
-      if (staged_aligned) {
+      if (!ANY || staged_aligned) {
         static_for<0, NP / PB>([&](auto b) {
           i32x4_t x[PB];
           static_for<0, PB>([&](auto q) {
@@ -1644,7 +1652,7 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
           });
           asm volatile("; staged output block, fp16");
         }
-      } else if (d.out.ptr != nullptr) {
+      } else if (ANY && d.out.ptr != nullptr) {
         static_for<0, NJ>([&](auto j) { store_out16(d.out, mw + 32 * j, nw + 32 * i, M, N, A[j]); });
       }
       // Partial reductions exclude every element outside [0,M) x [0,N) (the
@@ -1785,7 +1793,7 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
       // 16 passes unrolled: their LDS reads are in flight together (measured 2%
       // faster than 4 at 16384x4096x1024 with no ops; the kernel's code is small
       // enough since the column blocks share one copy of the op code).
-      if (out_flags & kFlagAligned) {
+      if (!ANY || (out_flags & kFlagAligned)) {
 #pragma unroll 16
         for (int p = 0; p < BM / RPP; ++p) {
           const int rl = p * RPP + crow;
@@ -1810,7 +1818,7 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
       }
       // Row ends that are no whole chunk, in the tile that holds them: element
       // by element, a row per thread.
-      if ((N & 7) != 0 && n0 + BN > N) {
+      if (ANY && (N & 7) != 0 && n0 + BN > N) {
         const int ce = (N - n0) >> 3;
         for (int rl = tid; rl < BM; rl += NT) {
           const int m = m0 + rl;
@@ -1875,11 +1883,14 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
 
 // Explicit instantiation of one tile variant's four generic kernels (bf16/f16
 // operands, with and without reductions), and of fixed-chain kernels.
-#define FUSEML_GEMM_INSTANTIATE_ONE(C, T, R, CH)                                                  \
+#define FUSEML_GEMM_INSTANTIATE_ANY(C, T, R, CH, ANY)                                              \
   template __global__ void fuseml_gemm::gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, \
-                                                              C.sched, T, R, CH>(const fuseml_gemm_desc);
-#define FUSEML_GEMM_INSTANTIATE(C)                                             \
-  FUSEML_GEMM_INSTANTIATE_ONE(C, __bf16, false, fuseml_gemm::kChainGeneric)    \
-  FUSEML_GEMM_INSTANTIATE_ONE(C, __bf16, true, fuseml_gemm::kChainGeneric)     \
-  FUSEML_GEMM_INSTANTIATE_ONE(C, _Float16, false, fuseml_gemm::kChainGeneric)  \
-  FUSEML_GEMM_INSTANTIATE_ONE(C, _Float16, true, fuseml_gemm::kChainGeneric)
+                                                              C.sched, T, R, CH, ANY>(const fuseml_gemm_desc);
+#define FUSEML_GEMM_INSTANTIATE_ONE(C, T, R, CH) FUSEML_GEMM_INSTANTIATE_ANY(C, T, R, CH, true)
+// The generic kernels of one value of ANY.
+#define FUSEML_GEMM_INSTANTIATE_ROWS(C, ANY)                                          \
+  FUSEML_GEMM_INSTANTIATE_ANY(C, __bf16, false, fuseml_gemm::kChainGeneric, ANY)      \
+  FUSEML_GEMM_INSTANTIATE_ANY(C, __bf16, true, fuseml_gemm::kChainGeneric, ANY)       \
+  FUSEML_GEMM_INSTANTIATE_ANY(C, _Float16, false, fuseml_gemm::kChainGeneric, ANY)    \
+  FUSEML_GEMM_INSTANTIATE_ANY(C, _Float16, true, fuseml_gemm::kChainGeneric, ANY)
+#define FUSEML_GEMM_INSTANTIATE(C) FUSEML_GEMM_INSTANTIATE_ROWS(C, true)

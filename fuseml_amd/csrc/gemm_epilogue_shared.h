@@ -38,6 +38,15 @@ constexpr TileConfig kNarrow32 = {32, 128, 64, 3, 1, 4, 0};  // 4 waves lock-ste
 constexpr TileConfig kLarge128 = {256, 128, 32, 4, 4, 2, 1};  // 8 waves ping-pong (wave tile 64x64), 100 KB LDS, 1 WG/CU
 constexpr TileConfig kSmall64 = {128, 128, 64, 4, 2, 2, 0};  // kSmall at BK = 64: 130 KB LDS, 1 WG/CU
 
+// Whether a variant has a kernel of its own for aligned rows (parameter ANY): the
+// tiles below 256x256, whose prologue and epilogue are the larger share.  Without the
+// code for ragged rows they take (M x N x K, bf16, us, one kernel -> two)
+// 2048x1024x4096 bias+residual 30.35 -> 29.93, 2048x1024x1024 bias+GELU 12.39 ->
+// 12.25, 2048x2048x1024 bias+residual 17.98 -> 17.87, 2048x1024x1024 ReLU + three row
+// reductions 13.93 -> 13.73; the 256x256 ping-pong kernel 4096x4096x768 bias+residual
+// 36.20 -> 36.02 but 4096x4096x512 bias+GELU 29.19 -> 29.48, so that one stays single.
+constexpr bool splits_rows(const TileConfig& c) { return c.bm * c.bn < 256 * 256; }
+
 // Launch tile `index` of kKsplit; T: __bf16, _Float16 or float GEMM operands
 // (gemm_ksplit_v_*.hip).
 template <typename T>
@@ -66,7 +75,7 @@ enum FixedChain : int {
 // The kernel (defined in gemm_epilogue_kernel.h).  SCHED selects the K-loop
 // schedule, T the GEMM operand type (__bf16 or _Float16), RED whether the
 // launch has reductions, CH the epilogue chain (FixedChain).
-template <int BM, int BN, int BK, int S, int WM, int WN, int SCHED, typename T, bool RED, int CH>
+template <int BM, int BN, int BK, int S, int WM, int WN, int SCHED, typename T, bool RED, int CH, bool ANY>
 __global__ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg);
 
 }  // namespace fuseml_gemm

@@ -3,4 +3,5 @@
 // library's kernels compile in parallel.
 #include "gemm_epilogue_kernel.h"
 
-FUSEML_GEMM_INSTANTIATE(fuseml_gemm::kLarge128)
+FUSEML_GEMM_INSTANTIATE_ROWS(fuseml_gemm::kLarge128, false)
+FUSEML_GEMM_INSTANTIATE_ROWS(fuseml_gemm::kLarge128, true)

@@ -3,5 +3,7 @@
 // the library's kernels compile in parallel.
 #include "gemm_epilogue_kernel.h"
 
-FUSEML_GEMM_INSTANTIATE(fuseml_gemm::kNarrow64)
-FUSEML_GEMM_INSTANTIATE(fuseml_gemm::kNarrow32)
+FUSEML_GEMM_INSTANTIATE_ROWS(fuseml_gemm::kNarrow64, false)
+FUSEML_GEMM_INSTANTIATE_ROWS(fuseml_gemm::kNarrow64, true)
+FUSEML_GEMM_INSTANTIATE_ROWS(fuseml_gemm::kNarrow32, false)
+FUSEML_GEMM_INSTANTIATE_ROWS(fuseml_gemm::kNarrow32, true)

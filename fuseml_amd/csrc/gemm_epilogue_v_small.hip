@@ -3,5 +3,7 @@
 // compile in parallel.
 #include "gemm_epilogue_kernel.h"
 
-FUSEML_GEMM_INSTANTIATE(fuseml_gemm::kSmall)
-FUSEML_GEMM_INSTANTIATE(fuseml_gemm::kSmall64)
+FUSEML_GEMM_INSTANTIATE_ROWS(fuseml_gemm::kSmall, false)
+FUSEML_GEMM_INSTANTIATE_ROWS(fuseml_gemm::kSmall, true)
+FUSEML_GEMM_INSTANTIATE_ROWS(fuseml_gemm::kSmall64, false)
+FUSEML_GEMM_INSTANTIATE_ROWS(fuseml_gemm::kSmall64, true)

@@ -50,15 +50,17 @@ PROBE_KERNEL_HINT = "mfma_peak_kernel"
 
 
 def _short(name: str) -> str:
-    """gemm_epilogue_kernel<BM,BN,BK,S,WM,WN,SCHED,dtype[,red][,chN]> from the
-    mangled name (",red": the instantiation that carries the reductions;
-    ",chN": fixed epilogue chain N, absent for the generic op loop, chain 0)."""
-    m = re.search(r"gemm_epilogue_kernelI((?:Li\d+E)+)(DF16b|DF16_)(?:Lb([01])E)?(?:Li(\d+)E)?E", name)
+    """gemm_epilogue_kernel<BM,BN,BK,S,WM,WN,SCHED,dtype[,red][,chN][,aligned]> from
+    the mangled name (",red": the instantiation that carries the reductions;
+    ",chN": fixed epilogue chain N, absent for the generic op loop, chain 0;
+    ",aligned": the one without the code for ragged rows)."""
+    m = re.search(r"gemm_epilogue_kernelI((?:Li\d+E)+)(DF16b|DF16_)(?:Lb([01])E)?(?:Li(\d+)E)?(?:Lb([01])E)?E", name)
     if m:
         ints = ",".join(re.findall(r"Li(\d+)E", m.group(1)))
         dtype = {"DF16b": "bf16", "DF16_": "f16"}[m.group(2)]
         ch = f",ch{m.group(4)}" if m.group(4) not in (None, "0") else ""
-        return f"gemm_epilogue_kernel<{ints},{dtype}{',red' if m.group(3) == '1' else ''}{ch}>"
+        rows = ",aligned" if m.group(5) == "0" else ""
+        return f"gemm_epilogue_kernel<{ints},{dtype}{',red' if m.group(3) == '1' else ''}{ch}{rows}>"
     # Demangled by the profiler: "void ns::gemm_epilogue_kernel<256, 256, ..., __bf16, true, 3>(...)".
     # rocprofv3 demangles some instantiations with a garbled type tail (the
     # __bf16 mangling); then only the seven tile integers are kept.
@@ -67,11 +69,12 @@ def _short(name: str) -> str:
         ints = m.group(1).replace(" ", "")
         tail = [t.strip() for t in m.group(2).split(",")]
         dtype = {"__bf16": "bf16", "_Float16": "f16"}.get(tail[0]) if tail else None
-        if dtype is None or len(tail) not in (2, 3) or tail[1] not in ("true", "false") or \
-                (len(tail) == 3 and not tail[2].isdigit()):
+        if dtype is None or len(tail) not in (2, 3, 4) or tail[1] not in ("true", "false") or \
+                (len(tail) >= 3 and not tail[2].isdigit()) or (len(tail) == 4 and tail[3] not in ("true", "false")):
             return f"gemm_epilogue_kernel<{ints},...>"
-        ch = f",ch{tail[2]}" if len(tail) == 3 and tail[2] != "0" else ""
-        return f"gemm_epilogue_kernel<{ints},{dtype}{',red' if tail[1] == 'true' else ''}{ch}>"
+        ch = f",ch{tail[2]}" if len(tail) >= 3 and tail[2] != "0" else ""
+        rows = ",aligned" if tail[3:] == ["false"] else ""
+        return f"gemm_epilogue_kernel<{ints},{dtype}{',red' if tail[1] == 'true' else ''}{ch}{rows}>"
     return name[:60]
 
 

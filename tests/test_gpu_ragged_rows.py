@@ -100,3 +100,28 @@ def test_column_reductions_with_staged_tiles(variant, shape):
     _check_red(mean, ref["mean"], np.abs(v).mean(axis=0), "mean")
     # tighter than the contract's 1e-2: fp32 sums of M values
     assert np.allclose(_np(s), ref["sum"], rtol=1e-4)
+
+
+@pytest.mark.parametrize("out", ["bf16", "fp32", "none"])
+@pytest.mark.parametrize("first,second", [("contiguous", "contiguous"), ("contiguous", "offset1"), ("offset1", "contiguous")])
+def test_aligned_and_ragged_launches(variant, first, second, out):
+    """Two 2-D operands, each aligned or not, beside a staged output, one that is not
+    staged and none (an escape store and a reduction instead): the kernel without the
+    code for ragged rows runs where nothing needs it, and only there."""
+    M, N, K, dtype = 150, 264, 72, torch.bfloat16
+    a, w = _gemm_inputs(M, N, K, dtype, seed=67)
+    views = _residual_views(M, N, dtype)
+    inputs = [views[first], views[second], a.cuda(), w.t().cuda()]
+    steps = [("add", 0, 1.0), ("mul", 1, 1.0), ("relu", -1, 1.0)]
+    print(f"case aligned and ragged {variant} {first} {second} {out}", flush=True)
+    spec = dict(left=2, right=3, ops=steps, out_dtype=torch.float32 if out == "fp32" else dtype, reductions=("sum",),
+                reduce_axis=1, reduce_dtypes=(torch.float32,), outputs=(("tile",), ("red", "sum")))
+    if out == "none":
+        spec |= dict(ops=steps[:2] + [("store", 0, 1.0)] + steps[2:], store_tile=False, extra_dtypes=(dtype,),
+                     outputs=(("extra", 0), ("red", "sum")))
+    tile, s = _launcher(_spec(**spec), 4)(*inputs)
+    torch.cuda.synchronize()
+    values = [_np(t) for t in inputs]
+    ref = ora.gemm_epilogue(values, 2, 3, steps, ("sum",), 1)
+    _check_tile(tile, ora.gemm_epilogue(values, 2, 3, steps[:2])["tile"] if out == "none" else ref["tile"])
+    _check_red(s, ref["sum"], np.abs(ref["tile"]).sum(axis=1), "sum")

@@ -130,6 +130,19 @@ def test_kernel_names_demangled_by_the_profiler():
     assert _short(garbled) == "gemm_epilogue_kernel<256,256,64,2,2,2,6,...>"
 
 
+def test_kernel_names_of_aligned_rows():
+    """The last template argument: false for the kernel without the code for ragged rows."""
+    from fuseml_amd.profiling import _short
+
+    base = "_ZN11fuseml_gemm20gemm_epilogue_kernelILi64ELi128ELi64ELi3ELi2ELi2ELi0E"
+    name = "gemm_epilogue_kernel<64,128,64,3,2,2,0,bf16"
+    assert _short(base + "DF16bLb0ELi0ELb0EEEv16fuseml_gemm_desc") == name + ",aligned>"
+    assert _short(base + "DF16bLb1ELi0ELb1EEEv16fuseml_gemm_desc") == name + ",red>"
+    dem = "void fuseml_gemm::gemm_epilogue_kernel<64, 128, 64, 3, 2, 2, 0, __bf16, "
+    assert _short(dem + "true, 0, false>(fuseml_gemm_desc)") == name + ",red,aligned>"
+    assert _short(dem + "false, 8, true>(fuseml_gemm_desc)") == name + ",ch8>"
+
+
 def test_counter_summary_means_per_launch_and_wave(tmp_path):
     """`counters` averages each counter per (kernel, launch) and per wave of the grid."""
     from fuseml_amd.profiling import counter_summary
