@@ -63,14 +63,20 @@ def _run(cmd: list[str], verbose: bool) -> None:
 
 
 def fastcall_command(out: str) -> list[str]:
-    """The host compiler's line for the CPython extension of the launchers."""
+    """The host compiler's line for the CPython extension of the launchers.
+
+    NDEBUG: pybind11's headers hold a thread-local counter without it, and an
+    extension with thread-local storage that no call touches makes every access to
+    other libraries' thread-locals take glibc's slow path (a module loaded later has
+    raised the generation that __tls_get_addr compares): 12% of the host time of each
+    torch operation in the process."""
     import sysconfig
 
     import torch
     from torch.utils.cpp_extension import include_paths
 
     lib = os.path.join(os.path.dirname(torch.__file__), "lib")
-    return [os.environ.get("CXX") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+    return [os.environ.get("CXX") or "g++", "-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{INCLUDE_DIR}",
             *[a for p in include_paths() for a in ("-isystem", p)], f"-I{sysconfig.get_paths()['include']}",
             os.path.join(CSRC_DIR, "fastcall.cpp"), "-o", out, f"-L{lib}", "-ltorch_python", "-ltorch", "-ltorch_cpu",

@@ -5,6 +5,7 @@ two on the device; the rest needs none.
 
 from __future__ import annotations
 
+import struct
 import threading
 
 import pytest
@@ -52,6 +53,20 @@ def test_malformed_plans_are_refused(bad):
     except ValueError:
         return
     assert checked_late and taken is False
+
+
+def test_the_extension_has_no_thread_local_storage():
+    """Its ELF program headers hold no PT_TLS (7): see build.fastcall_command."""
+    from fuseml_amd.build import FASTCALL_PATH
+
+    with open(FASTCALL_PATH, "rb") as f:
+        head = f.read(64)
+        offset, = struct.unpack_from("<Q", head, 32)
+        size, count = struct.unpack_from("<HH", head, 54)
+        f.seek(offset)
+        table = f.read(size * count)
+    assert head[:5] == b"\x7fELF\x02"
+    assert 7 not in [struct.unpack_from("<I", table, size * i)[0] for i in range(count)]
 
 
 gpu = pytest.mark.gpu
