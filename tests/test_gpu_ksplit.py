@@ -24,6 +24,7 @@ SHAPES = [
     ((17, 1030, 1000), (16, 32, 4)),    # N % 4 != 0, K ends inside a chunk
     ((100, 257, 4640), (16, 16, 8)),    # odd N
     ((16, 256, 72), (16, 32, 4)),
+    ((128, 256, 1024), (16, 32, 4)),    # the reference's small preset's second GEMM
     ((30, 4112, 520), (32, 16, 4)),
     ((63, 4099, 520), (32, 32, 4)),
     ((8, 16384, 264), (16, 64, 4)),

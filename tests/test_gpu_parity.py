@@ -220,13 +220,13 @@ def test_variant_chain_parity(forced_variant, chain, shape):
 # The automatic tile choice on the device (its CU count): one shape per tile it
 # picks below a full round of 256x256 tiles, and a 64-row output with a full
 # round of them (M <= 128 runs on the smaller tiles).  The launched tile is
-# asserted through fuseml_gemm_epilogue_config, the output checked against
-# the oracle on two chains (one with a 2-D operand).
+# asserted through fuseml_gemm_epilogue_config (which speaks for the tiled family:
+# that the K-split kernel does not take the shape is asserted beside it), the output
+# checked against the oracle on two chains (one with a 2-D operand).
 AUTO_TILES = [
     ((2048, 4096, 256), (256, 128, 8)),   # 256 ping-pong tiles: one round
     ((2048, 1024, 256), (64, 128, 4)),
     ((1000, 1000, 256), (32, 128, 4)),    # ragged M and N
-    ((128, 256, 1024), (32, 128, 4)),     # the reference's small preset's second GEMM
     ((64, 65536, 256), (64, 128, 4)),     # 64 rows against a wide weight: one row of 64x128 tiles
     ((100, 33000, 264), (128, 128, 4)),   # 100 rows: one row of 128x128 tiles at BK = 64, ragged N and K
     ((4096, 4096, 256), (256, 256, 8)),   # a full round: the 256x256 ping-pong kernel
@@ -257,6 +257,7 @@ def test_automatic_tile_choice_parity(shape, tile, chain):
     lib = _abi.load_library()
     assert lib.fuseml_gemm_epilogue_config(plan.desc_ref, cfg) == 0, _abi.last_error(lib)
     assert tuple(cfg[:3]) == tile, (shape, tuple(cfg[:3]))
+    assert lib.fuseml_gemm_epilogue_ksplit(plan.desc_ref, cfg) == 0
     ref = ora.gemm_epilogue([_np(t) for t in inputs], left, right, steps)["tile"]
     _check_tile(out, ref, f"auto {shape} {chain}")
 
