@@ -1695,10 +1695,10 @@ void gemm_epilogue_kernel(const fuseml_gemm_desc d_arg) {
         } else if (col_red) {
           // Column partials: first over this lane's row blocks, then over the 32
           // rows of its half-wave by halving: at lane distance 16, 8, 4 and 2 a
-          // lane hands over the half of its columns that its partner keeps, so 16
-          // exchanges (and one more at distance 1) leave every lane with the sum
+          // lane hands over the half of its columns that its partner keeps, so 15
+          // exchanges and one more at distance 1 leave every lane with the sum
           // of one column, r = (l32 >> 1), where a full exchange of each column
-          // takes 80.  The 16x fewer values stay in registers until the output
+          // takes 80 (and as many for the maximum).  The 16x fewer values stay in registers until the output
           // is drained, so the output and a 2-D operand are staged in LDS as they
           // are beside row reductions (16384x4096x1024 ReLU + three column
           // reductions, bf16: 227.7 -> 165.1 us; over rows 137.0).

@@ -157,7 +157,9 @@ int fuseml_gemm_epilogue_supported(const fuseml_gemm_desc* desc);
  * waves per workgroup and LDS bytes into cfg[0..3].  Replaces the launch
  * parameter selection of kernel_launcher.py:134-306 / sram_autotuner.py.  It
  * speaks for the tiled family; a small output may run on the K-split kernel
- * instead (fuseml_gemm_epilogue_ksplit). */
+ * instead (fuseml_gemm_epilogue_ksplit).  This query, _ksplit and _chain describe
+ * `desc` as one launch: an output of a little more than whole rounds of 256x256
+ * tiles runs as two, the whole rounds and the rest, each chosen for its own size. */
 int fuseml_gemm_epilogue_config(const fuseml_gemm_desc* desc, int32_t cfg[4]);
 
 /* Whether a launch of `desc` runs on the K-split kernel (few output tiles, the
