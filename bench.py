@@ -8,7 +8,8 @@ workload (default C2, the MLP block: GEMM1+bias+GELU and GEMM2+bias+residual,
 two launches of the gfx950 kernel family through the C ABI) on synthetic
 seeded inputs resident in HBM.  W untimed steps, then exactly K timed steps
 bracketed by ``torch.cuda.synchronize()``; ``value`` = wall ms per step.
-Rank 0 prints one JSON line carrying:
+Rank 0 prints one JSON line carrying (of ``configs`` and ``reference_presets`` the
+times, speedups and check results; the records whole go to stderr):
 
 * ``roofline`` — the dominant kernel's algorithmic FLOPs per launch over its
   average launch duration (HIP events on the launch stream, inside the timed
@@ -1010,7 +1011,32 @@ def main():
         "fp32_block": fp32,
         "cpu_baseline": cpu,
     }
+    details = {k: line[k] for k in ("configs", "reference_presets")}
+    print(f"[bench] details {json.dumps(details)}", file=sys.stderr, flush=True)
+    line["configs"], line["reference_presets"] = _summaries(configs), _summaries(presets)
     print(json.dumps(line), flush=True)
+
+
+def _summaries(records):
+    """The figures of each config's or preset's record that the result line carries:
+    per measured form its time, the speedup over eager and the device's time where
+    that was measured, and whether every check passed.  The whole records, some
+    20 KB, are longer than a reader of the output's last part sees."""
+    if not records:
+        return records
+    out = {}
+    for name, r in records.items():
+        forms = {k: v for k, v in r.items() if isinstance(v, dict) and "median_ms" in v}
+        checks = [f["check"].get("ok", f["check"].get("pass")) for f in forms.values() if f.get("check")]
+        s = out[name] = {k: r[k] for k in ("speedup_vs_eager", "dominant_frac_spec") if k in r}
+        s["ok"] = all(checks) if checks else None
+        for k, f in forms.items():
+            s[k] = {"ms": f["median_ms"]}
+            if "speedup_vs_eager" in f:
+                s[k]["speedup_vs_eager"] = f["speedup_vs_eager"]
+            if f.get("device"):
+                s[k]["device_ms"] = f["device"]["device_ms"]
+    return out
 
 
 def _gemms_of(name):

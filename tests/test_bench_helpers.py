@@ -2,6 +2,7 @@
 per launch and the fused-against-eager traffic from the committed summaries."""
 
 import importlib.util
+import json
 import os
 
 import torch
@@ -110,3 +111,25 @@ def test_preset_roofline_names_the_binding_roofline():
     t = bench.preset_traffic("mlp_block", M, D, I, 1)
     r = bench.preset_roofline(0.03, 2 * 2.0 * M * D * I, t["compulsory_bytes"])
     assert r["bound"] == "mfma"
+
+
+def test_result_line_summaries_are_short():
+    """The records' times, speedups and checks, a fraction of their length."""
+    bench = _bench()
+    check = {"rows_checked": 66, "ok": True, "tile_max_abs_err": 0.007737159729003906}
+    form = {"median_ms": 0.2325, "p25_ms": 0.2316, "p75_ms": 0.2336, "iters": 4140, "check": check, "tflops": 1182.3}
+    preset = form | {"check": {"max_abs_err": 0.0145, "pass": True}, "speedup_vs_eager": 2.4, "dispatch": ["direct"],
+                     "device": {"device_ms": 0.0089, "tflops": 15.1, "frac_mfma": 0.006, "bound": "hbm"}}
+    records = {
+        "C4": {"workload": "a long description " * 8, "fused": form, "fused_cold": {"median_ms": 0.238, "iters": 9},
+               "kernels": [{"kernel": "k", "avg_ms": 0.2}], "speedup_vs_eager": 1.6, "dominant_frac_spec": 0.47},
+        "small": {"workload": "mlp_block", "M": 128, "eager": form, "compiled": preset, "all_fused": None}}
+    got = bench._summaries(records)
+    assert got["C4"] == {"speedup_vs_eager": 1.6, "dominant_frac_spec": 0.47, "ok": True, "fused": {"ms": 0.2325},
+                         "fused_cold": {"ms": 0.238}}
+    assert got["small"] == {"ok": True, "eager": {"ms": 0.2325},
+                            "compiled": {"ms": 0.2325, "speedup_vs_eager": 2.4, "device_ms": 0.0089}}
+    preset["check"]["pass"] = False
+    assert bench._summaries(records)["small"]["ok"] is False
+    assert len(json.dumps(got)) < len(json.dumps(records)) / 3
+    assert bench._summaries({}) == {} and bench._summaries(None) is None
