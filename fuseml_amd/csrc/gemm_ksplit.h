@@ -141,8 +141,9 @@ __device__ __forceinline__ void convert_raw4(const Op& op, i32x4_t x, float v[4]
 }
 
 // MB x NB blocks of 16 rows x 16 columns per tile; NW waves split K; DEPTH
-// chunks of 128 bytes of every row per wave in its LDS ring.
-template <int MB, int NB, int NW, int DEPTH, typename T>
+// chunks of 128 bytes of every row per wave in its LDS ring.  RED: the launch has
+// reductions; the others' kernels carry none of that code (3% of a 6 us launch).
+template <int MB, int NB, int NW, int DEPTH, typename T, bool RED>
 __global__ __launch_bounds__(NW * 64) void gemm_ksplit_kernel(const fuseml_gemm_desc d_arg) {
   constexpr int BM = 16 * MB, BN = 16 * NB, NT = NW * 64;
   constexpr int UNITS = BM * BN / 4;             // runs of 4 columns
@@ -287,16 +288,18 @@ __global__ __launch_bounds__(NW * 64) void gemm_ksplit_kernel(const fuseml_gemm_
   }
   lds_barrier();
 
-  // A unit's values into the fused reductions.  The BN / 4 units of a row are
-  // neighbouring lanes, the units of a column lie BN / 4 lanes apart; one atomic
-  // per row of the tile, or per column and wave.  Elements outside [0, M) x
-  // [0, N) never enter.
-  auto reduce = [&](const float v[4], int m, int n, int nq, int lane) {
-    auto put = [&](int idx, float s, float mx, float inv) {
-      if (d.reduce_mask & FUSEML_RED_SUM) atomicAdd(d.reduce_out[0] + idx, s);
-      if (d.reduce_mask & FUSEML_RED_AMAX) atomic_max_f32(d.reduce_out[1] + idx, mx);
-      if (d.reduce_mask & FUSEML_RED_MEAN) atomicAdd(d.reduce_out[2] + idx, s * inv);
-    };
+  // A unit's values into the fused reductions, one atomic per row or column of the
+  // tile.  The BN / 4 units of a row are neighbouring lanes.  A thread's units all
+  // lie in the same 4 columns, whose partials it keeps to the end (col_s, col_mx).
+  // Elements outside [0, M) x [0, N) never enter.
+  auto put = [&](int idx, float s, float mx, float inv) {
+    if (d.reduce_mask & FUSEML_RED_SUM) atomicAdd(d.reduce_out[0] + idx, s);
+    if (d.reduce_mask & FUSEML_RED_AMAX) atomic_max_f32(d.reduce_out[1] + idx, mx);
+    if (d.reduce_mask & FUSEML_RED_MEAN) atomicAdd(d.reduce_out[2] + idx, s * inv);
+  };
+  static_assert(NT % (BN / 4) == 0, "a thread's units share their columns");
+  float col_s[4] = {0.0f, 0.0f, 0.0f, 0.0f}, col_mx[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+  auto reduce = [&](const float v[4], int m, int n, int nq) {
     float s[4], mx[4];
     static_for<0, 4>([&](auto e) {
       const bool in = m < M && n + e < N;
@@ -313,18 +316,10 @@ __global__ __launch_bounds__(NW * 64) void gemm_ksplit_kernel(const fuseml_gemm_
       }
       if (nq == 0 && m < M) put(m, s[0], mx[0], 1.0f / (float)N);
     } else {
-#pragma unroll
-      for (int sh = BN / 4; sh < 64; sh <<= 1) {
-        static_for<0, 4>([&](auto e) {
-          s[e] += __shfl_xor(s[e], sh);
-          mx[e] = max_nan(mx[e], __shfl_xor(mx[e], sh));
-        });
-      }
-      if (lane < BN / 4) {
-        static_for<0, 4>([&](auto e) {
-          if (n + e < N) put(n + e, s[e], mx[e], 1.0f / (float)M);
-        });
-      }
+      static_for<0, 4>([&](auto e) {
+        col_s[e] += s[e];
+        col_mx[e] = max_nan(col_mx[e], mx[e]);
+      });
     }
   };
 
@@ -369,8 +364,41 @@ __global__ __launch_bounds__(NW * 64) void gemm_ksplit_kernel(const fuseml_gemm_
       }
     }
     if (d.out.ptr != nullptr) store_out4(d.out, m, n, M, N, v);
-    if (d.reduce_mask != 0) reduce(v, m, n, nq, lane);
+    if constexpr (RED) reduce(v, m, n, nq);
   });
+
+  // Column partials: over the lanes of the wave that hold the same columns (BN / 4
+  // apart), then over the waves through LDS, where every wave has read the K
+  // partials by the first barrier.  (With one atomic per column and wave step
+  // instead, M / 4 on each column at BN = 64, 824x528x4480 ReLU + three column
+  // reductions took 54.6 us for 16.9, 29.1 on the tiled kernels.)
+  if (RED && d.reduce_axis == 0) {
+#pragma unroll
+    for (int sh = BN / 4; sh < 64; sh <<= 1) {
+      static_for<0, 4>([&](auto e) {
+        col_s[e] += __shfl_xor(col_s[e], sh);
+        col_mx[e] = max_nan(col_mx[e], __shfl_xor(col_mx[e], sh));
+      });
+    }
+    lds_barrier();
+    float* part_s = reinterpret_cast<float*>(smem);
+    float* part_mx = part_s + NW * BN;
+    if (lane < BN / 4) {
+      static_for<0, 4>([&](auto e) {
+        part_s[wave * BN + 4 * lane + e] = col_s[e];
+        part_mx[wave * BN + 4 * lane + e] = col_mx[e];
+      });
+    }
+    lds_barrier();
+    if (tid < BN && n0 + tid < N) {
+      float s = 0.0f, mx = -INFINITY;
+      static_for<0, NW>([&](auto w) {
+        s += part_s[w * BN + tid];
+        mx = max_nan(mx, part_mx[w * BN + tid]);
+      });
+      put(n0 + tid, s, mx, 1.0f / (float)M);
+    }
+  }
 }
 
 template <int I, typename T>
@@ -379,8 +407,11 @@ void launch_ksplit_tile(const fuseml_gemm_desc& d, int index, hipStream_t stream
     constexpr KsplitConfig C = kKsplit[I];
     if (index != I) return launch_ksplit_tile<I + 1, T>(d, index, stream);
     const int64_t tiles = ((d.M + C.bm() - 1) / C.bm()) * ((d.N + C.bn() - 1) / C.bn());
-    hipLaunchKernelGGL((gemm_ksplit_kernel<C.mb, C.nb, C.waves, C.depth, T>), dim3((unsigned)tiles),
-                       dim3(C.waves * 64), 0, stream, d);
+    const dim3 grid((unsigned)tiles), block(C.waves * 64);
+    if (d.reduce_mask != 0)
+      hipLaunchKernelGGL((gemm_ksplit_kernel<C.mb, C.nb, C.waves, C.depth, T, true>), grid, block, 0, stream, d);
+    else
+      hipLaunchKernelGGL((gemm_ksplit_kernel<C.mb, C.nb, C.waves, C.depth, T, false>), grid, block, 0, stream, d);
   }
 }
 
