@@ -210,9 +210,9 @@ def runs_ksplit(M: int, N: int, K: int, cus: int = MI355X_CUS) -> bool:
         tiles = -(-M // (16 * mb)) * -(-N // (16 * nb))
         alone = waves * 2 * 16 * (mb + nb) * 128 > 80 * 1024  # one workgroup per CU
         fixed = 5.1 if alone else 0.6 if mb * nb == 2 else 1.2
-        least = min(least, (1.0 if alone else 3.5) + max(1.0, tiles / cus) * (fixed + 0.32 * (mb + nb) * K / 1024))
+        least = min(least, (1.0 if alone else 3.5) + -(-tiles // cus) * (fixed + 0.36 * (mb + nb) * K / 1024))
     tiled = -3.0 + partial_round_tile(M, N, K, cus)[1] / 160.0 * (5.05 + 3.6 * K / 1024)
-    return least < 0.85 * tiled
+    return least < 0.9 * tiled
 
 
 def ksplit_beats_eager(M: int, N: int, K: int) -> bool:

@@ -193,19 +193,25 @@ TileConfig choose_config(const fuseml_gemm_desc& d, int cus) {
 
 // The K-split tile (index into kKsplit) a launch of `d` runs on, or -1 for the
 // tiled family.  Both sides are priced in microseconds by what was measured on
-// 326 shapes of 1 to 2048 rows, 256 to 16384 columns and K = 256 to 16384 (bf16,
-// bias + residual), where the tiled family would run one of its tiles below a
-// round:
-//   K-split  3.5 + r (0.6 to 1.2 + 0.32 (mb + nb) K / 1024), r = tiles per CU, at
-//            least 1: launch, first loads, partials and epilogue, then operand
-//            bytes.  The 96 KB rings of the 32x64 and 64x32 tiles leave one
-//            workgroup per CU, so a further round overlaps nothing: 1 + r (5.1 + ..).
+// 1400 shapes of 1 to 2048 rows, 128 to 16384 columns and K = 64 to 16384, most of
+// them ragged (bf16: bias + residual, bias + GELU, ReLU + three row or column
+// reductions), where the tiled family would run one of its tiles below a round:
+//   K-split  3.5 + r (0.6 to 1.2 + 0.36 (mb + nb) K / 1024), r the rounds of a tile
+//            per CU: launch, first loads, partials and epilogue, then operand bytes.
+//            Whole rounds, since the CU with the most tiles ends last: 257 tiles
+//            take nearly as long as 512.  The 96 KB rings of the 32x64 and 64x32
+//            tiles leave one workgroup per CU, so a further round overlaps nothing:
+//            1 + r (5.1 + ..).
 //   tiled    -3 + work (5.05 + 3.6 K / 1024) / 160, work as choose_partial_round
 //            weighs it.
-// Each is within 8% of the measurement on average, 33% at worst, so the K-split
-// kernel runs where it is priced at 0.85 of the other or less: 227 of the 326
-// shapes, 2.0x faster there (geometric mean; 0.15-0.97 of the tiled time), e.g.
-// 8x4096x16384 107.7 -> 27.0, 64x4096x4096 31.4 -> 14.3, 128x256x1024 10.3 -> 5.1.
+//   both     fused reductions (reduction_us).
+// The K-split price is within 17% of the measurement on average, so that kernel runs
+// where it is priced at 0.9 of the other or less: 1097 of the 1400 shapes, 1.9x
+// faster there (geometric mean), 2 of them slower than the tiled family by more than
+// 2% (353x192x64 with row reductions 7.9 -> 9.4, 1371x720x5728 36.7 -> 39.9); e.g.
+// 8x4096x16384 107.7 -> 27.0, 64x4096x4096 31.4 -> 14.3, 128x256x1024 10.3 -> 5.1.  With tiles /
+// CUs for r, 0.32 and 0.85 it took 1150, 34 of them slower: 182x2944x1024 10.8 ->
+// 14.6, 1808x416x4728 30.8 -> 39.5, 1069x992x7600 51.9 -> 76.9.
 // Not at 1024x1024x1024 (11.0 tiled, 13.0 here: operands shared by more waves
 // win) nor where the weight streams through a full row of tiles
 // (16x65536x1024 28.5 against 30.7).
@@ -213,11 +219,15 @@ int choose_ksplit(const fuseml_gemm_desc& d, int cus) {
   if (forced_variant() != 0 || d.K <= 0 || weight_streaming(d, cus)) return -1;
   if (d.M > 128 && 2 * cdiv(d.M, 256) * cdiv(d.N, 256) > cus) return -1;
   double cost = 0.0;
-  const int best = cheapest_ksplit(d.M, d.N, d.K, cus, 0.32, &cost);
+  const int best = cheapest_ksplit(d.M, d.N, d.K, cus, kKsplitPerK, &cost);
   int64_t work = 0;
   choose_partial_round(d, cus, &work);
-  const double tiled = -3.0 + (double)work / (5.0 * 160.0) * (5.05 + 3.6 * (double)d.K / 1024.0);
-  return cost < 0.85 * tiled ? best : -1;
+  double tiled = -3.0 + (double)work / (5.0 * 160.0) * (5.05 + 3.6 * (double)d.K / 1024.0);
+  if (d.reduce_mask != 0) {
+    cost += reduction_us(d.reduce_axis == 1, d.M, d.N, kKsplit[best].bn());
+    tiled += reduction_us(d.reduce_axis == 1, d.M, d.N, 128);
+  }
+  return cost < kKsplitMargin * tiled ? best : -1;
 }
 
 int choose_ksplit_f32(const fuseml_gemm_desc& d, int cus) { return ksplit_f32(d.M, d.N, d.K, cus); }
@@ -621,9 +631,9 @@ bool split_rounds(fuseml_gemm_desc& d, int cus, fuseml_gemm_desc& rest) {
   double small = 0.0;
   int64_t work = 0;
   choose_partial_round(r, cus, &work);
-  cheapest_ksplit(r.M, r.N, r.K, cus, 0.32, &small);
+  cheapest_ksplit(r.M, r.N, r.K, cus, kKsplitPerK, &small);
   const double tiled = -3.0 + (double)work / (5.0 * 160.0) * (5.05 + 3.6 * k);
-  if (small >= 0.85 * tiled) small = tiled;
+  if (small >= kKsplitMargin * tiled) small = tiled;
   if (small + 2.0 > 0.9 * partial) return false;
   derive_flags(r);
   rest = r;

@@ -25,14 +25,26 @@ constexpr KsplitConfig kKsplit[] = {{1, 1, 8, 2}, {1, 2, 4, 2}, {2, 1, 4, 2}, {2
                                     {1, 4, 4, 2}, {2, 4, 4, 2}, {4, 2, 4, 2}};
 constexpr int kNumKsplit = 7;
 
+// us per block row or column of a tile and 1024 of K, 16-bit operands.
+constexpr double kKsplitPerK = 0.36;
+// The K-split kernel runs where it is priced at this part of the tiled family or less.
+constexpr double kKsplitMargin = 0.9;
+
+// us that fused reductions add on tiles of `bn` columns.  Over columns 2 on either
+// side.  Over rows 1, and one atomic per row and column tile, of which those of 32
+// rows queue on one line of the output, about 1.5 ns each (16x8128x2544 ReLU + three
+// row reductions on 32 columns 17.1 us, 6.5 without).
+inline double reduction_us(bool rows, int64_t M, int64_t N, int bn) {
+  return rows ? 1.0 + 0.0015 * (double)((N + bn - 1) / bn) * (double)(M < 32 ? M : 32) : 2.0;
+}
+
 // The K-split tile with the least priced time (the formula is choose_ksplit's, in
 // gemm_epilogue.hip), `per_k` us per block row or column and 1024 of K.
 inline int cheapest_ksplit(int64_t M, int64_t N, int64_t K, int cus, double per_k, double* least) {
   int best = -1;
   for (int i = 0; i < kNumKsplit; ++i) {
     const KsplitConfig& c = kKsplit[i];
-    const double tiles = (double)c.tiles(M, N);
-    const double r = tiles > cus ? tiles / cus : 1.0;
+    const double r = (double)((c.tiles(M, N) + cus - 1) / cus);
     const bool alone = c.lds_bytes() > 80 * 1024;
     const double fixed = alone ? 5.1 : c.mb * c.nb == 2 ? 0.6 : 1.2;
     const double t = (alone ? 1.0 : 3.5) + r * (fixed + per_k * (c.mb + c.nb) * (double)K / 1024.0);

@@ -25,11 +25,12 @@ SHAPES = [
     ((100, 257, 4640), (16, 16, 8)),    # odd N
     ((16, 256, 72), (16, 32, 4)),
     ((128, 256, 1024), (16, 32, 4)),    # the reference's small preset's second GEMM
-    ((30, 4112, 520), (32, 16, 4)),
-    ((63, 4099, 520), (32, 32, 4)),
-    ((8, 16384, 264), (16, 64, 4)),
+    ((90, 1355, 2312), (32, 16, 4)),
+    ((500, 507, 520), (32, 32, 4)),
+    ((255, 1001, 1032), (32, 32, 4)),
+    ((8, 16384, 1544), (16, 64, 4)),
     ((500, 1023, 2056), (32, 64, 4)),
-    ((1000, 520, 2056), (64, 32, 4)),
+    ((950, 530, 2056), (64, 32, 4)),
 ]
 _ID = lambda v: "x".join(map(str, v))  # noqa: E731
 
