@@ -45,10 +45,10 @@ MLP_CHUNK = 32
 # fill the chip (at least one per CU) and the weights are small (D = 256):
 # 0.84-0.92x of the two launches' time at M >= 16384 on 256 CUs (0.98x at
 # M = 65536, I = 1024), 1.04-1.74x below that; D = 512 loses (1.06-1.41x) and
-# D = 1024 too (2.24x).  Those are the four-wave kernel's; on the eight-wave one
-# D = 256 measures 0.71-0.92x from M = 16384, 0.81-0.88x at 8192 (32-row blocks;
-# the rule still leaves it to two launches), 1.10-1.19x below, and D = 512
-# 0.90-1.03x.
+# D = 1024 too (2.24x).  Those rows are the four-wave kernel's, as is the rule; on
+# the eight-wave one the same sweep gives D = 256 0.70-0.92x from M = 16384,
+# 0.83-0.86x at 8192 (32-row blocks; the rule still leaves it to two launches),
+# 1.09-1.21x below, and D = 512 0.89-1.02x.
 MLP_AUTO_WIDTH = 256
 MLP_AUTO_MIN_ROW_BLOCKS = 256
 
