@@ -451,25 +451,18 @@ int match_fixed_chain(const fuseml_gemm_desc& d) {
 
 // `max_wg` caps the grid (0: one workgroup per tile); the kernel loops over the
 // remaining tiles.
-template <const TileConfig& C, bool ANY>
+template <const TileConfig& C, typename T, bool ANY>
 hipError_t launch_rows(const fuseml_gemm_desc& d, hipStream_t stream, int max_wg) {
   int64_t tiles = cdiv(d.M, C.bm) * cdiv(d.N, C.bn);
   if (max_wg > 0 && tiles > max_wg) tiles = max_wg;
   const dim3 grid((unsigned)tiles), block(C.wm * C.wn * 64);
-  const bool red = d.reduce_mask != 0;
   constexpr int G = kChainGeneric;
-  if (d.ab_dtype == FUSEML_BF16 && !red)
-    hipLaunchKernelGGL((gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, C.sched, __bf16, false, G, ANY>),
-                       grid, block, 0, stream, d);
-  else if (d.ab_dtype == FUSEML_BF16)
-    hipLaunchKernelGGL((gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, C.sched, __bf16, true, G, ANY>),
-                       grid, block, 0, stream, d);
-  else if (!red)
-    hipLaunchKernelGGL((gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, C.sched, _Float16, false, G, ANY>),
-                       grid, block, 0, stream, d);
+  if (d.reduce_mask == 0)
+    hipLaunchKernelGGL((gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, C.sched, T, false, G, ANY>), grid,
+                       block, 0, stream, d);
   else
-    hipLaunchKernelGGL((gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, C.sched, _Float16, true, G, ANY>),
-                       grid, block, 0, stream, d);
+    hipLaunchKernelGGL((gemm_epilogue_kernel<C.bm, C.bn, C.bk, C.stages, C.wm, C.wn, C.sched, T, true, G, ANY>), grid,
+                       block, 0, stream, d);
   return hipGetLastError();
 }
 
@@ -483,12 +476,18 @@ bool needs_any(const fuseml_gemm_desc& d) {
   return d.out.ptr != nullptr && (d.out.reserved & kBoth) != kBoth;
 }
 
+template <const TileConfig& C, typename T>
+hipError_t launch_typed(const fuseml_gemm_desc& d, hipStream_t stream, int max_wg) {
+  if constexpr (splits_rows<T>(C)) {
+    if (!needs_any(d)) return launch_rows<C, T, false>(d, stream, max_wg);
+  }
+  return launch_rows<C, T, true>(d, stream, max_wg);
+}
+
 template <const TileConfig& C>
 hipError_t launch_variant(const fuseml_gemm_desc& d, hipStream_t stream, int max_wg) {
-  if constexpr (splits_rows(C)) {
-    if (!needs_any(d)) return launch_rows<C, false>(d, stream, max_wg);
-  }
-  return launch_rows<C, true>(d, stream, max_wg);
+  return d.ab_dtype == FUSEML_BF16 ? launch_typed<C, __bf16>(d, stream, max_wg)
+                                   : launch_typed<C, _Float16>(d, stream, max_wg);
 }
 
 // A fixed-chain kernel of variant C (reductions only with kChainRelu, as

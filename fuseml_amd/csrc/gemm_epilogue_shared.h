@@ -9,6 +9,8 @@
 
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "fuseml_hip.h"
 #include "ksplit_rule.h"
 
@@ -43,9 +45,14 @@ constexpr TileConfig kSmall64 = {128, 128, 64, 4, 2, 2, 0};  // kSmall at BK = 6
 // code for ragged rows they take (M x N x K, bf16, us, one kernel -> two)
 // 2048x1024x4096 bias+residual 30.35 -> 29.93, 2048x1024x1024 bias+GELU 12.39 ->
 // 12.25, 2048x2048x1024 bias+residual 17.98 -> 17.87, 2048x1024x1024 ReLU + three row
-// reductions 13.93 -> 13.73; the 256x256 ping-pong kernel 4096x4096x768 bias+residual
-// 36.20 -> 36.02 but 4096x4096x512 bias+GELU 29.19 -> 29.48, so that one stays single.
-constexpr bool splits_rows(const TileConfig& c) { return c.bm * c.bn < 256 * 256; }
+// reductions 13.93 -> 13.73.  The 256x256 ping-pong kernel has one for fp16 alone:
+// 689x11288x576 bias+GELU, scale, add 27.74 -> 26.98 (26.93 before ragged rows were
+// staged), its other chains 0.99-1.01; in bf16 that chain had lost nothing, and
+// bias+GELU would lose 1% (28.59 -> 28.87 at 4096x4096x576).
+template <typename T>
+constexpr bool splits_rows(const TileConfig& c) {
+  return c.bm * c.bn < 256 * 256 || (c.sched == kLarge.sched && std::is_same<T, _Float16>::value);
+}
 
 // Launch tile `index` of kKsplit; T: __bf16, _Float16 or float GEMM operands
 // (gemm_ksplit_v_*.hip).
